@@ -108,6 +108,8 @@ int prefill_key_splits(int P, int pos0, int window, int n_kv_heads, int group, i
 int prefill_tile_keys(int head_dim);
 size_t prefill_tile_bytes(int head_dim);
 
+// The combine of ksplit > 1 partials (also made by launch_prefill_attn).
+hipError_t launch_prefill_combine(const pk::PrefillArgs& a, int head_dim, int ksplit, hipStream_t stream);
 // Plain 16-byte-per-thread copy kernel.
 hipError_t launch_copy(void* dst, const void* src, size_t bytes, hipStream_t stream);
 

@@ -90,6 +90,13 @@ hipError_t launch_attn_d(const pk::PrefillArgs& a, int group, const uint4* ws, i
 
 template <int D>
 hipError_t launch_combine_d(const pk::PrefillArgs& a, int ksplit, hipStream_t stream) {
+    const long long cols = (long long)a.P * a.Hq * (D / 4);
+    if (ksplit <= 8 && cols >= 512 * pk::kCombineThreads) {   // enough blocks for two per CU
+        hipLaunchKernelGGL((pk::prefill_combine_rows_kernel<D>),
+                           dim3((unsigned)((cols + pk::kCombineThreads - 1) / pk::kCombineThreads)),
+                           dim3(pk::kCombineThreads), 0, stream, a, ksplit);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL((pk::prefill_combine_kernel<D>), dim3((unsigned)(a.P * a.Hq)),
                        dim3(pk::kCombineThreads), 0, stream, a, ksplit);
     return hipGetLastError();
@@ -190,6 +197,10 @@ hipError_t launch_prefill_attn(const pk::PrefillArgs& a, int head_dim, int group
     default: return hipErrorInvalidValue;
     }
     if (e != hipSuccess || ksplit <= 1) return e;
+    return launch_prefill_combine(a, head_dim, ksplit, stream);
+}
+
+hipError_t launch_prefill_combine(const pk::PrefillArgs& a, int head_dim, int ksplit, hipStream_t stream) {
     switch (head_dim) {
     case 64: return launch_combine_d<64>(a, ksplit, stream);
     case 96: return launch_combine_d<96>(a, ksplit, stream);

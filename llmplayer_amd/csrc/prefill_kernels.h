@@ -441,44 +441,49 @@ __device__ __forceinline__ int wave_max_int(int x) {
     return __builtin_amdgcn_readfirstlane(x);
 }
 
-// Query fragment of one lane for MFMA B operands: dims 32*s + 8*grp + j of query token qi
-// (clamped into range), head hq, as fp32 (or widened from bf16), QK-normed, rotated, scaled,
-// then split.  NEOX partners (d, d + half) usually sit in other lanes, so each element reads
-// its partner from the input and normalises it exactly as the partner's own lane does; any
-// rotated width (partial RoPE) works the same way.  The scaled queries of the wave are divided
+// Eight consecutive values from a 16-byte aligned address.
+__device__ __forceinline__ void load8(const float* p, float (&v)[8]) {
+    const float4 x0 = reinterpret_cast<const float4*>(p)[0], x1 = reinterpret_cast<const float4*>(p)[1];
+    v[0] = x0.x; v[1] = x0.y; v[2] = x0.z; v[3] = x0.w;
+    v[4] = x1.x; v[5] = x1.y; v[6] = x1.z; v[7] = x1.w;
+}
+// Eight consecutive bf16 values, widened.  (The prompt arrays need only their element's
+// alignment, which the hardware's 16-byte loads take.)
+__device__ __forceinline__ void load8_bf16(const unsigned short* p, float (&v)[8]) {
+    const uint4 w = *reinterpret_cast<const uint4*>(p);
+    const unsigned u[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        v[2 * j] = __uint_as_float(u[j] << 16);
+        v[2 * j + 1] = __uint_as_float(u[j] & 0xFFFF0000u);
+    }
+}
+
+// Query fragment of one lane for MFMA B operands of STEP rows (32: four lane groups of 16, 16:
+// two of 32): dims STEP*s + 8*grp + j of query token qi (clamped into range), head hq, as fp32 (or widened from bf16), QK-normed, rotated, scaled,
+// then split.  With every dim rotated a NEOX pair (d, d + D/2) sits in one lane (but for head_dim
+// 96 in steps of 32); otherwise each element reads its partner from the input and normalises it exactly as the partner's own
+// lane does.  (A branch and a load per element cost one round trip each: 700 tokens at the
+// 16/8/128 shape with QK-norm took 69.3 us per call, 37.8 without.)  The scaled queries of the wave are divided
 // by 2^eq before their split, eq the range exponent of the largest magnitude among them (0
 // below 2^15; wave-uniform, so the factor that restores the scores stays in scalar registers);
 // the scores are multiplied back.
-template <int D>
+template <int D, int STEP = 32>
 __device__ __forceinline__ void query_fragment(const PrefillArgs& a, int qi, int hq, int qpos,
-                                               int grp, f16x8 (&qh)[D / 32],
-                                               f16x8 (&ql)[D / 32], int& eq) {
-    constexpr int KS = D / 32;
+                                               int grp, f16x8 (&qh)[D / STEP],
+                                               f16x8 (&ql)[D / STEP], int& eq) {
+    constexpr int KS = D / STEP;
     float qf[KS][8];
     const long long q0 = (long long)qi * a.Hq * D + (long long)hq * D;
-    // A lane's 8 elements per step are contiguous and 16-byte aligned (D is a multiple of 32):
-    // one 16-byte load per step for bf16 inputs, two for fp32.
+    // A lane's 8 elements per step are contiguous: one 16-byte load per step for bf16 inputs, two
+    // for fp32.  (Every branch of this prologue stands outside its loop over the steps: a step's
+    // loads behind a branch wait for their own round trip, 1.5-2 us each here.)
     if (a.in_f32) {
-        const float* qp = static_cast<const float*>(a.q) + q0;
 #pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            const float4 x0 = *reinterpret_cast<const float4*>(qp + 32 * s + 8 * grp);
-            const float4 x1 = *reinterpret_cast<const float4*>(qp + 32 * s + 8 * grp + 4);
-            qf[s][0] = x0.x; qf[s][1] = x0.y; qf[s][2] = x0.z; qf[s][3] = x0.w;
-            qf[s][4] = x1.x; qf[s][5] = x1.y; qf[s][6] = x1.z; qf[s][7] = x1.w;
-        }
+        for (int s = 0; s < KS; ++s) load8(static_cast<const float*>(a.q) + q0 + STEP * s + 8 * grp, qf[s]);
     } else {
-        const unsigned short* qp = static_cast<const unsigned short*>(a.q) + q0;
 #pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            const uint4 w = *reinterpret_cast<const uint4*>(qp + 32 * s + 8 * grp);
-            const unsigned u[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                qf[s][2 * j] = __uint_as_float(u[j] << 16);
-                qf[s][2 * j + 1] = __uint_as_float(u[j] & 0xFFFF0000u);
-            }
-        }
+        for (int s = 0; s < KS; ++s) load8_bf16(static_cast<const unsigned short*>(a.q) + q0 + STEP * s + 8 * grp, qf[s]);
     }
     float r = 1.0f;
     if (a.qnw != nullptr) {
@@ -487,66 +492,95 @@ __device__ __forceinline__ void query_fragment(const PrefillArgs& a, int qi, int
         for (int s = 0; s < KS; ++s)
 #pragma unroll
             for (int j = 0; j < 8; ++j) ss = __builtin_fmaf(qf[s][j], qf[s][j], ss);
-        ss = dk::lane_step<16, false>(ss);
+        if constexpr (STEP == 32) ss = dk::lane_step<16, false>(ss);
         ss = dk::lane_step<32, false>(ss);
         r = 1.0f / sqrtf(ss / (float)D + a.eps);
 #pragma unroll
-        for (int s = 0; s < KS; ++s)
+        for (int s = 0; s < KS; ++s) {
+            float wv[8];
+            load8(a.qnw + STEP * s + 8 * grp, wv);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) qf[s][j] = (qf[s][j] * r) * a.qnw[32 * s + 8 * grp + j];
+            for (int j = 0; j < 8; ++j) qf[s][j] = (qf[s][j] * r) * wv[j];
+        }
     }
     if (a.cos_t != nullptr) {
         const float* cr = a.cos_t + (long long)qpos * a.half_rope;
         const float* sr = a.sin_t + (long long)qpos * a.half_rope;
         const int half = a.half_rope;
-        if (a.rope_type == 0) {
-#pragma unroll
-            for (int s = 0; s < KS; ++s) {
-                // the lane's 4 pairs are consecutive table entries: one 16-byte load each for
-                // cos and sin when all 4 rotate and the rows are 16-byte aligned
-                const int i0 = 16 * s + 4 * grp;
-                float cv[4], sv[4];
-                if ((half & 3) == 0 && i0 + 3 < half) {
-                    const float4 c4 = *reinterpret_cast<const float4*>(cr + i0);
-                    const float4 s4 = *reinterpret_cast<const float4*>(sr + i0);
-                    cv[0] = c4.x; cv[1] = c4.y; cv[2] = c4.z; cv[3] = c4.w;
-                    sv[0] = s4.x; sv[1] = s4.y; sv[2] = s4.z; sv[3] = s4.w;
-                } else {
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        const bool rot = i0 + u < half;
-                        cv[u] = cr[rot ? i0 + u : 0];
-                        sv[u] = sr[rot ? i0 + u : 0];
-                    }
-                }
+        if (a.rope_type == 0) {   // pairs (2i, 2i + 1): the lane's 4 pairs are consecutive table entries
+            auto rotate = [&](float (&x)[8], const float (&cv)[4], const float (&sv)[4], int i0) {
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
-                    const int j = 2 * u;
                     const bool rot = i0 + u < half;
-                    const float c = cv[u], sn = sv[u];
-                    const float v0 = qf[s][j], v1 = qf[s][j + 1];
-                    const float t0 = v0 * c, t1 = v1 * sn, t2 = v0 * sn, t3 = v1 * c;
-                    qf[s][j] = rot ? t0 - t1 : v0;
-                    qf[s][j + 1] = rot ? t2 + t3 : v1;
+                    const float v0 = x[2 * u], v1 = x[2 * u + 1];
+                    const float t0 = v0 * cv[u], t1 = v1 * sv[u], t2 = v0 * sv[u], t3 = v1 * cv[u];
+                    x[2 * u] = rot ? t0 - t1 : v0;
+                    x[2 * u + 1] = rot ? t2 + t3 : v1;
+                }
+            };
+            if (2 * half == D) {   // all dims rotate: rows of D/2 floats, one 16-byte load each
+#pragma unroll
+                for (int s = 0; s < KS; ++s) {
+                    const int i0 = STEP / 2 * s + 4 * grp;
+                    const float4 c4 = *reinterpret_cast<const float4*>(cr + i0);
+                    const float4 s4 = *reinterpret_cast<const float4*>(sr + i0);
+                    const float cv[4] = {c4.x, c4.y, c4.z, c4.w}, sv[4] = {s4.x, s4.y, s4.z, s4.w};
+                    rotate(qf[s], cv, sv, i0);
+                }
+            } else {
+#pragma unroll
+                for (int s = 0; s < KS; ++s) {
+                    const int i0 = STEP / 2 * s + 4 * grp;
+                    float cv[4], sv[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        cv[u] = cr[min(i0 + u, half - 1)];
+                        sv[u] = sr[min(i0 + u, half - 1)];
+                    }
+                    rotate(qf[s], cv, sv, i0);
                 }
             }
         } else {  // NEOX: pairs (i, i + half) for i < half; dims >= 2*half keep their values
+            if (D % (2 * STEP) == 0 && 2 * half == D) {
+                // Every dim rotates and the partner of the lane's (step s, j) is its own
+                // (s + KS/2, j): no loads but the table rows'.
+                constexpr int KH = KS / 2;
 #pragma unroll
-            for (int s = 0; s < KS; ++s)
+                for (int s = 0; s < KH; ++s) {
+                    float cv[8], sv[8];
+                    load8(cr + STEP * s + 8 * grp, cv);
+                    load8(sr + STEP * s + 8 * grp, sv);
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int d = 32 * s + 8 * grp + j;
-                    if (d < 2 * half) {
-                        const bool first = d < half;
-                        const int i = first ? d : d - half, pd = first ? d + half : d - half;
-                        float pv = in_val(a.q, q0 + pd, a.in_f32);
-                        if (a.qnw != nullptr) pv = (pv * r) * a.qnw[pd];
-                        const float v0 = first ? qf[s][j] : pv, v1 = first ? pv : qf[s][j];
-                        const float c = cr[i], sn = sr[i];
-                        const float t0 = v0 * c, t1 = v1 * sn, t2 = v0 * sn, t3 = v1 * c;
-                        qf[s][j] = first ? t0 - t1 : t2 + t3;
+                    for (int j = 0; j < 8; ++j) {
+                        const float v0 = qf[s][j], v1 = qf[s + KH][j];
+                        const float t0 = v0 * cv[j], t1 = v1 * sv[j], t2 = v0 * sv[j], t3 = v1 * cv[j];
+                        qf[s][j] = t0 - t1;
+                        qf[s + KH][j] = t2 + t3;
                     }
                 }
+            } else {
+                // The partners are read from the input again, unconditionally (clamped), so that
+                // the loads are in flight together.
+                auto partial = [&](auto f32) {
+#pragma unroll
+                    for (int s = 0; s < KS; ++s)
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) {
+                            const int d = STEP * s + 8 * grp + j;
+                            const bool rot = d < 2 * half, first = d < half;
+                            const int pd = !rot ? 0 : first ? d + half : d - half;
+                            const int i = !rot ? 0 : first ? d : d - half;
+                            float pv = in_val(a.q, q0 + pd, decltype(f32)::value);
+                            const float c = cr[i], sn = sr[i];
+                            if (a.qnw != nullptr) pv = (pv * r) * a.qnw[pd];
+                            const float v0 = first ? qf[s][j] : pv, v1 = first ? pv : qf[s][j];
+                            const float t0 = v0 * c, t1 = v1 * sn, t2 = v0 * sn, t3 = v1 * c;
+                            qf[s][j] = !rot ? qf[s][j] : first ? t0 - t1 : t2 + t3;
+                        }
+                };
+                if (a.in_f32) partial(std::integral_constant<int, 1>{});
+                else partial(std::integral_constant<int, 0>{});
+            }
         }
     }
     float qmax = 0.0f;
@@ -1085,6 +1119,42 @@ __global__ __launch_bounds__(kCombineThreads) void prefill_combine_kernel(Prefil
         r.w = dk::finish_output(M, L, O.w, a.sinks, a.gate, hq, g0 + 3);
         reinterpret_cast<float4*>(a.out + row * D)[c] = r;
     }
+}
+
+// The same for few splits and many rows: one thread per (row, float4 column), the splits merged in
+// its registers, 256 / (D / 4) rows per block.  Bound by the partials' bytes; one block per row
+// had 16 of 256 threads loading at two splits (32/8/64, 512 tokens: 16.6 us; 16/8/128, 777 tokens: 9.1 us, 5.4 this way).
+template <int D>
+__global__ __launch_bounds__(kCombineThreads) void prefill_combine_rows_kernel(PrefillArgs a, int ksplit) {
+    constexpr int NC = D / 4;
+    const long long rows = (long long)a.P * a.Hq;
+    const long long e = (long long)blockIdx.x * kCombineThreads + threadIdx.x;
+    if (e >= rows * NC) return;
+    const long long row = e / NC;
+    const int c = (int)(e - row * NC), hq = (int)(row % a.Hq);
+    float m = kNegBig, l = 0.0f;
+    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+    for (int s = 0; s < ksplit; ++s) {
+        const long long slot = (long long)s * rows + row;
+        const float2 ml = *reinterpret_cast<const float2*>(a.part_ml + 2 * slot);
+        const float4 x = reinterpret_cast<const float4*>(a.part_o + slot * D)[c];
+        const float mn = fmaxf(m, ml.x);
+        const float so = dk::fast_exp2(m - mn), sx = dk::fast_exp2(ml.x - mn);
+        l = __builtin_fmaf(l, so, ml.y * sx);
+        o.x = __builtin_fmaf(o.x, so, x.x * sx);
+        o.y = __builtin_fmaf(o.y, so, x.y * sx);
+        o.z = __builtin_fmaf(o.z, so, x.z * sx);
+        o.w = __builtin_fmaf(o.w, so, x.w * sx);
+        m = mn;
+    }
+    const long long g0 = row * D + 4 * c;
+    float4 r;
+    r.x = dk::finish_output(m, l, o.x, a.sinks, a.gate, hq, g0);
+    r.y = dk::finish_output(m, l, o.y, a.sinks, a.gate, hq, g0 + 1);
+    r.z = dk::finish_output(m, l, o.z, a.sinks, a.gate, hq, g0 + 2);
+    r.w = dk::finish_output(m, l, o.w, a.sinks, a.gate, hq, g0 + 3);
+    reinterpret_cast<float4*>(a.out + row * D)[c] = r;
 }
 
 }  // namespace pk
