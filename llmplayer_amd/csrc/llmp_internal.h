@@ -110,6 +110,15 @@ size_t prefill_tile_bytes(int head_dim);
 
 // The combine of ksplit > 1 partials (also made by launch_prefill_attn).
 hipError_t launch_prefill_combine(const pk::PrefillArgs& a, int head_dim, int ksplit, hipStream_t stream);
+// The wide path (prefill_wide_kernels.h): its key splits for a call, 0 where the call stays on
+// the kernels above; keys and bytes per tile image; and its launches (images into `ws`,
+// attention, and with ksplit > 1 the combine).
+int prefill_wide_splits(int P, int pos0, int window, int n_kv_heads, int group, int head_dim, int n_cu);
+int prefill_wide_tile_keys(int head_dim);
+size_t prefill_wide_tile_bytes(int head_dim);
+hipError_t launch_prefill_wide(const pk::PrefillArgs& a, int head_dim, int group, void* ws, int tile0, int n_tiles,
+                               int row_end, int n_cu, hipStream_t stream);
+
 // Plain 16-byte-per-thread copy kernel.
 hipError_t launch_copy(void* dst, const void* src, size_t bytes, hipStream_t stream);
 

@@ -1778,58 +1778,55 @@ static int enqueue_prefill(KvHandle* kv, int layer, int src_layer, int pos0, int
     // Key tiles any query of this call attends: from the first query's window start (or 0) to
     // the last prompt row.  Their images live in the handle's workspace, grown when a call
     // needs more (a growth synchronises the device; the size only depends on the row range).
-    const int TK = prefill_tile_keys(D);
     const int kbeg_min = a.window > 0 ? std::max(0, pos0 - a.window + 1) : 0;
-    const int tile0 = kbeg_min / TK, tile_last = (pos0 + n_tokens - 1) / TK;
-    const int n_tiles = tile_last - tile0 + 1;
-    const int ksplit = prefill_key_splits(n_tokens, pos0, a.window, Hkv * c.krep, group, D, G().n_cu);
-    const size_t ws_bytes =
-        ksplit == 1 ? (size_t)Hkv * (size_t)n_tiles * prefill_tile_bytes(D) : 0;
-    const size_t part_bytes =
-        ksplit > 1
-            ? (size_t)ksplit * (size_t)n_tokens * (size_t)c.n_heads * (size_t)(D + 2) * sizeof(float)
-            : 0;
-    void* ws = nullptr;
+    int TK = prefill_tile_keys(D);
+    int tile0 = kbeg_min / TK;
+    int n_tiles = (pos0 + n_tokens - 1) / TK - tile0 + 1;
+    int ksplit = prefill_key_splits(n_tokens, pos0, a.window, Hkv * c.krep, group, D, G().n_cu);
+    const size_t part_1 = (size_t)n_tokens * (size_t)c.n_heads * (size_t)(D + 2) * sizeof(float);
+    size_t ws_bytes = ksplit == 1 ? (size_t)Hkv * (size_t)n_tiles * prefill_tile_bytes(D) : 0;
+    size_t part_bytes = ksplit > 1 ? (size_t)ksplit * part_1 : 0;
+    // The static array's limit counts this plan's workspace, on either path.
+    if (use_static && ws_bytes + part_bytes > (size_t)LLMP_PREFILL_STATIC_BYTES)
+        return fail(LLMP_ERR_INVALID_ARG,
+                    "llmp_attn_prefill_f32_static: the call needs %zu bytes of workspace; the "
+                    "static scratch holds %u (fewer tokens per call, or llmp_attn_prefill_f32)",
+                    ws_bytes + part_bytes, (unsigned)LLMP_PREFILL_STATIC_BYTES);
+    const int wide = prefill_wide_splits(n_tokens, pos0, a.window, Hkv * c.krep, group, D, G().n_cu);
+    bool use_wide = false;
+    if (wide > 0) {
+        const int wtk = prefill_wide_tile_keys(D), wt0 = kbeg_min / wtk;
+        const int wnt = (pos0 + n_tokens - 1) / wtk - wt0 + 1;
+        const size_t wws = KvHandle::pad256((size_t)Hkv * (size_t)wnt * prefill_wide_tile_bytes(D));
+        const size_t wpart = wide > 1 ? (size_t)wide * part_1 : 0;
+        if (!use_static || wws + wpart <= (size_t)LLMP_PREFILL_STATIC_BYTES) {
+            use_wide = true;
+            TK = wtk, tile0 = wt0, n_tiles = wnt, ksplit = wide, ws_bytes = wws, part_bytes = wpart;
+        }
+    }
+    void* ws = kv->prefill_ws;
     if (use_static) {
-        // The whole workspace (tile images, or split-K partials) in the static array: no
+        // The whole workspace (tile images, split-K partials) in the static array: no
         // allocation, no profiling events.
-        const size_t need = ksplit > 1 ? part_bytes : ws_bytes;
-        if (need > (size_t)LLMP_PREFILL_STATIC_BYTES)
-            return fail(LLMP_ERR_INVALID_ARG,
-                        "llmp_attn_prefill_f32_static: the call needs %zu bytes of workspace; the "
-                        "static scratch holds %u (fewer tokens per call, or llmp_attn_prefill_f32)",
-                        need, (unsigned)LLMP_PREFILL_STATIC_BYTES);
-        void* sp = G().scratch;
-        if (!sp) return fail(LLMP_ERR_NOT_INIT, "llmp_attn_prefill_f32_static: no scratch address");
-        if (ksplit > 1) {
-            a.part_o = static_cast<float*>(sp);
-            a.part_ml = a.part_o + (size_t)ksplit * n_tokens * c.n_heads * D;
-        } else {
-            ws = sp;
+        ws = G().scratch;
+        if (!ws) return fail(LLMP_ERR_NOT_INIT, "llmp_attn_prefill_f32_static: no scratch address");
+        a.part_o = reinterpret_cast<float*>(static_cast<char*>(ws) + ws_bytes);
+    } else {
+        if (ws_bytes > kv->prefill_ws_bytes) {
+            if (kv->prefill_ws) {
+                LLMP_HIP_CHECK(hipStreamSynchronize(st), "hipStreamSynchronize");
+                (void)hipFree(kv->prefill_ws);
+                kv->prefill_ws = nullptr;
+                kv->prefill_ws_bytes = 0;
+            }
+            hipError_t e = hipMalloc(&kv->prefill_ws, ws_bytes);
+            if (e == hipErrorOutOfMemory)
+                return fail(LLMP_ERR_OUT_OF_MEMORY, "llmp_attn_prefill: %zu-byte tile workspace", ws_bytes);
+            LLMP_HIP_CHECK(e, "hipMalloc(prefill workspace)");
+            kv->prefill_ws_bytes = ws_bytes;
         }
-        if (!shared) LLMP_HIP_CHECK(launch_prefill_append(a, D, st), "prefill append launch");
-        if (ksplit == 1)
-            LLMP_HIP_CHECK(launch_prefill_tiles(a, D, ws, tile0, n_tiles, pos0 + n_tokens, st),
-                           "prefill tile launch");
-        LLMP_HIP_CHECK(launch_prefill_attn(a, D, group, ws, tile0, n_tiles, G().n_cu, ksplit, st),
-                       "prefill attention launch");
-        return LLMP_OK;
-    }
-    if (ws_bytes > kv->prefill_ws_bytes) {
-        if (kv->prefill_ws) {
-            LLMP_HIP_CHECK(hipStreamSynchronize(st), "hipStreamSynchronize");
-            (void)hipFree(kv->prefill_ws);
-            kv->prefill_ws = nullptr;
-            kv->prefill_ws_bytes = 0;
-        }
-        hipError_t e = hipMalloc(&kv->prefill_ws, ws_bytes);
-        if (e == hipErrorOutOfMemory)
-            return fail(LLMP_ERR_OUT_OF_MEMORY, "llmp_attn_prefill: %zu-byte tile workspace", ws_bytes);
-        LLMP_HIP_CHECK(e, "hipMalloc(prefill workspace)");
-        kv->prefill_ws_bytes = ws_bytes;
-    }
-    // Key splits (short prompts after a long prefix) and their partials buffer.
-    if (ksplit > 1) {
+        ws = kv->prefill_ws;
+        // Key splits (chunks whose query blocks leave CUs idle) and their partials buffer.
         if (part_bytes > kv->prefill_part_bytes) {
             if (kv->prefill_part) {
                 LLMP_HIP_CHECK(hipStreamSynchronize(st), "hipStreamSynchronize");
@@ -1845,27 +1842,32 @@ static int enqueue_prefill(KvHandle* kv, int layer, int src_layer, int pos0, int
             kv->prefill_part_bytes = part_bytes;
         }
         a.part_o = kv->prefill_part;
-        a.part_ml = kv->prefill_part + (size_t)ksplit * n_tokens * c.n_heads * D;
     }
+    if (ksplit > 1) a.part_ml = a.part_o + (size_t)ksplit * n_tokens * c.n_heads * D;
+    const bool prof = kv->prof_on && !use_static;
     hipEvent_t e0 = nullptr, e1 = nullptr, e2 = nullptr, e3 = nullptr;
-    if (kv->prof_on) {
+    if (prof) {
         for (hipEvent_t* e : {&e0, &e1, &e2, &e3})
             if (int rc = prof_event(kv, e)) return rc;
         LLMP_HIP_CHECK(hipEventRecord(e0, st), "hipEventRecord");
     }
     if (!shared) LLMP_HIP_CHECK(launch_prefill_append(a, D, st), "prefill append launch");
-    if (kv->prof_on) {
+    if (prof) {
         LLMP_HIP_CHECK(hipEventRecord(e1, st), "hipEventRecord");
         kv->prof_pending[LLMP_PROF_PREFILL_APPEND].push_back({e0, e1});
         LLMP_HIP_CHECK(hipEventRecord(e2, st), "hipEventRecord");
     }
-    if (ksplit == 1)   // split launches stage straight from the cache (no images)
-        LLMP_HIP_CHECK(launch_prefill_tiles(a, D, kv->prefill_ws, tile0, n_tiles, pos0 + n_tokens, st),
-                       "prefill tile launch");
-    LLMP_HIP_CHECK(launch_prefill_attn(a, D, group, kv->prefill_ws, tile0, n_tiles, G().n_cu,
-                                       ksplit, st),
-                   "prefill attention launch");
-    if (kv->prof_on) {
+    if (use_wide) {
+        LLMP_HIP_CHECK(launch_prefill_wide(a, D, group, ws, tile0, n_tiles, pos0 + n_tokens, G().n_cu, st),
+                       "prefill attention launch");
+    } else {
+        if (ksplit == 1)   // split launches stage straight from the cache (no images)
+            LLMP_HIP_CHECK(launch_prefill_tiles(a, D, ws, tile0, n_tiles, pos0 + n_tokens, st),
+                           "prefill tile launch");
+        LLMP_HIP_CHECK(launch_prefill_attn(a, D, group, ws, tile0, n_tiles, G().n_cu, ksplit, st),
+                       "prefill attention launch");
+    }
+    if (prof) {
         LLMP_HIP_CHECK(hipEventRecord(e3, st), "hipEventRecord");
         kv->prof_pending[LLMP_PROF_PREFILL_ATTN].push_back({e2, e3});
     }

@@ -1,0 +1,90 @@
+"""GPU parity of the wide multi-token attention (prefill_wide_kernels.h) against P sequential
+decodes of the oracle, at the edges of its launch forms: blocks in pairs (even and odd counts),
+key halves with one and with several key splits, one block per workgroup (many blocks), ragged
+lengths, windows, soft-cap, sinks, partial RoPE, head_dim 96, and Q8_0 rows.
+
+Bar: output max-abs <= 1e-4 (and <= 1e-4 + 1e-3*|ref|), the cache bit-identical."""
+import numpy as np
+import pytest
+
+from llmplayer_amd import _lib
+from llmplayer_amd import hip_forward_pass as hfp
+from oracle import oracle as orc
+from tests import decode_cases as dc
+
+pytestmark = pytest.mark.gpu
+
+LLAMA, QWEN3, GEMMA2, GEMMA3 = hfp.ARCH_LLAMA, hfp.ARCH_QWEN3, hfp.ARCH_GEMMA2, hfp.ARCH_GEMMA3
+
+# (hq, hkv, d, arch, extra ModelConfig fields, layer, pos0, P, QK-norm, sinks)
+CASES = {
+    "halves, one split": (24, 8, 128, LLAMA, {}, 0, 0, 1000, False, False),
+    "halves, full grid": (24, 8, 128, LLAMA, {}, 0, 37, 1301, False, False),
+    "pairs, odd block count": (24, 8, 128, LLAMA, {}, 0, 5, 1560, False, False),
+    "one block per workgroup": (32, 8, 64, LLAMA, {}, 0, 3, 2101, False, False),
+    "halves, key splits": (24, 8, 128, LLAMA, {}, 0, 3001, 97, False, False),
+    "group 2, QK-norm, NEOX": (16, 8, 128, QWEN3, {}, 0, 1501, 777, True, False),
+    "group 8, sinks": (64, 8, 64, LLAMA, {}, 0, 61, 701, False, True),
+    "window, soft-cap": (16, 4, 128, GEMMA2, {"sliding_window": 300, "attn_logit_soft_cap": 50.0},
+                         1, 90, 1403, False, False),
+    "window shorter than a tile": (32, 8, 64, GEMMA3, {"sliding_window": 20}, 0, 700, 4100, True, False),
+    "head_dim 96, NEOX": (32, 32, 96, LLAMA, {"rope_type": _lib.LLMP_ROPE_NEOX}, 0, 0, 1001, False, False),
+    "partial NEOX": (24, 8, 128, LLAMA, {"rope_type": _lib.LLMP_ROPE_NEOX, "rope_dim_count": 40}, 0, 11,
+                     900, True, False),
+    "partial pairs": (24, 8, 128, LLAMA, {"rope_dim_count": 52}, 0, 0, 900, False, False),
+}
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_wide_prefill_matches_sequential_decodes(name):
+    hq, hkv, d, arch, extra, layer, pos0, P, qkn, sinks = CASES[name]
+    c = hfp.ModelConfig(hq, hkv, d, layer + 1, architecture=arch, rope_freq_base=500000.0, **extra)
+    rng = np.random.default_rng(77 + P)
+    max_seq = pos0 + P
+    kc = np.zeros((max_seq, c.kv_dim), np.float32)
+    vc = np.zeros_like(kc)
+    kc[:pos0] = rng.standard_normal((pos0, c.kv_dim), dtype=np.float32)
+    vc[:pos0] = rng.standard_normal((pos0, c.kv_dim), dtype=np.float32)
+    q, k, v = (rng.standard_normal((P, n), dtype=np.float32) for n in (c.q_dim, c.kv_dim, c.kv_dim))
+    qk = tuple(rng.uniform(0.5, 1.5, d).astype(np.float32) for _ in range(2)) if qkn else None
+    sk = rng.standard_normal(hq).astype(np.float32) if sinks else None
+    with hfp.HipForwardPass(c, max_seq, qk_norm=[qk] * c.block_count if qkn else None,
+                            sinks=[sk] * c.block_count if sinks else None) as fp:
+        fp.kv.write(layer, 0, kc, vc)
+        dc.log(f"[gpu] wide prefill {name}: {hq}/{hkv}/{d} pos0={pos0} P={P}")
+        got = fp.prefill(layer, pos0, q, k, v)
+        cs, sn = dc.oracle_tables(c, max_seq, layer)
+        qw, kw = qk if qk is not None else (None, None)
+        want = orc.prefill_sequential(dc.oracle_config(c, max_seq, sk), kc, vc, q, k, v, layer, pos0,
+                                      qnorm_w=qw, knorm_w=kw, rope_cos=cs, rope_sin=sn, n_threads=16)
+        dc.compare_out(got.reshape(-1), want.reshape(-1), name)
+        dc.compare_cache(fp, layer, kc, vc, name + " cache")
+
+
+def test_wide_prefill_over_q8_rows_equals_dequantised_rows():
+    """Q8_0 rows and the same values in an fp32 cache give the same attention: the images hold
+    quant * scale either way, and the new rows' values are the quantised ones in both."""
+    c = hfp.ModelConfig(24, 8, 128, 1, architecture=LLAMA, rope_freq_base=500000.0)
+    pos0, P = 2000, 300
+    rng = np.random.default_rng(5)
+    nb = c.kv_dim // 32
+    qs = [rng.integers(-127, 128, (pos0, c.kv_dim), dtype=np.int8) for _ in range(2)]
+    sc = [rng.uniform(0.005, 0.02, (pos0, nb)).astype(np.float32) for _ in range(2)]
+    q, k, v = (rng.standard_normal((P, n), dtype=np.float32) for n in (c.q_dim, c.kv_dim, c.kv_dim))
+    with hfp.HipForwardPass(c, pos0 + P, kv_dtype=_lib.LLMP_KV_Q8_0) as f8, hfp.HipForwardPass(c, pos0 + P) as f32:
+        f8.kv.write_q8(0, 0, qs[0], sc[0], qs[1], sc[1])
+        got = f8.prefill(0, pos0, q, k, v)
+        kq, ks, vq, vs = f8.kv.read_q8(0, 0, pos0 + P)
+        rows = [(a.reshape(-1, nb, 32).astype(np.float32) * s[..., None]).reshape(-1, c.kv_dim)
+                for a, s in ((kq, ks), (vq, vs))]
+        f32.kv.write(0, 0, *rows)
+        # the same queries over the same values, as a shared-KV call: nothing is appended
+        dq, do = hfp.DeviceBuffer(q.nbytes), hfp.DeviceBuffer(q.nbytes)
+        try:
+            dq.upload(q)
+            _lib.call("llmp_attn_prefill_shared_f32", f32.kv.handle, 0, 0, pos0, P, dq.ptr, 0, do.ptr, 0)
+            want = do.download(np.float32, q.size)
+        finally:
+            dq.free()
+            do.free()
+    np.testing.assert_array_equal(got.reshape(-1), want)
