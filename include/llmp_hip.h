@@ -396,23 +396,26 @@ int llmp_attn_block(uint64_t handle, int layer, int position, uint64_t d_positio
                     int splits, uint64_t stream);
 
 /* The attention half of n_tokens consecutive tokens (positions pos0 .. pos0+n_tokens-1) on the
- * device residual rows x (fp32 [n_tokens][dim], 16-byte aligned, updated in place): what
- * n_tokens llmp_attn_block calls compute, with each projection weight read once per group of
- * up to 16 tokens (a group of one token runs the single-token call, which is faster for one
- * token).  Replaces LLMEngine.forwardBatch's per-token attention halves
- * (LLMEngine.java:1019-1033), batched as docs/optimization/speculative-decoding.md:120-140
- * plans for the verification of K draft tokens.  The projections run on the matrix cores with
- * each fp32 input split into two fp16 parts (fp32-accurate products, fp32 sums in another order
- * than the CPU path); any finite residual is taken: the inputs of a group are scaled by a power
- * of two that brings the largest below 2^15 (a small first kernel computes it with each token's
+ * device residual rows x (fp32 [n_tokens][dim], 16-byte aligned, updated in place): what n_tokens
+ * llmp_attn_block calls compute, with each projection weight read once per group of up to 16
+ * tokens (a group of one token runs the single-token call, which is faster for one token), or
+ * from 136 tokens on, in the fp32 input mode, as one product tiled by 128 tokens.  Replaces
+ * LLMEngine.forwardBatch's per-token attention halves (LLMEngine.java:1019-1033), batched as
+ * docs/optimization/speculative-decoding.md:120-140 plans for the verification of K draft tokens.
+ * The projections run on the matrix cores with each fp32 input split into two fp16 parts
+ * (fp32-accurate products, fp32 sums in another order than the CPU path); any finite residual is
+ * taken: the inputs of a group (of a token, in the tiled product) are scaled by a power of two
+ * that fits the largest to fp16's range (a small first kernel computes it with each token's
  * RMSNorm factor), the outputs by its inverse.  The attention is llmp_attn_prefill_f32's (the
  * appended rows bit-identical to single-token appends of the same projections).  In the
- * LLMP_INPUT_Q8_1 mode the routed types take each token's Q8_1 input as llmp_attn_block
- * forms it (the same staged norm and quantiser) and exact integer block dots on the matrix
- * cores, and Wo the quantised attention output.  At head_dim 80 (no prefill kernel) and for
- * layers whose fp32 or bf16 weights reach 65504, the tokens run one llmp_attn_block call each.  The call may grow the
- * handle's prefill workspace, as llmp_attn_prefill_f32 does (not for use under graph capture
- * then). */
+ * LLMP_INPUT_Q8_1 mode the routed types take each token's Q8_1 input as llmp_attn_block forms it
+ * (the same staged norm and quantiser) and exact integer block dots on the matrix cores, and Wo
+ * the quantised attention output.  At head_dim 80 (no prefill kernel) and for layers whose fp32
+ * or bf16 weights reach 65504, the tokens run one llmp_attn_block call each.  A call of up to 16
+ * tokens may grow the handle's prefill workspace, as llmp_attn_prefill_f32 does (not for use
+ * under graph capture then); longer ones have a scratch and workspaces of their own, which grow
+ * too: outgrown ones are kept until the handle is destroyed, so graphs captured before stay
+ * valid, and a captured call whose scratch would have to grow runs in groups of 16 tokens. */
 int llmp_attn_block_batch(uint64_t handle, int layer, int pos0, int n_tokens, uint64_t x,
                           uint64_t stream);
 

@@ -150,7 +150,7 @@ struct ProjTokArgs;
 // launch (second_type < 0: one type); hipErrorInvalidValue for an unsupported type or shape.
 // Per-token factors of a token-batched projection (tk::tok_prep_kernel): sc[2t] = the RMSNorm
 // factor r (1 without norm_w) and sc[2t + 1] = the range exponent of the largest x*w (or x),
-// for t < n_tokens (<= kTokBatch).
+// for t < n_tokens.
 hipError_t launch_tok_prep(const float* x, long long x_pitch, int cols, const float* norm_w, float eps,
                            float* sc, int n_tokens, hipStream_t stream);
 bool proj_tok_supported(int ggml_type);
@@ -160,9 +160,23 @@ bool proj_tok_pair_supported(int first_type, int second_type);
 hipError_t launch_proj_tok(const tk::ProjTokArgs& a, int first_type, int second_type, bool q8,
                            hipStream_t stream);
 bool proj_tok_q8_routed(int ggml_type);
+// Many-token projections (proj_gemm_kernels.h): the row exponents of an uploaded matrix (rows a
+// multiple of 16), the split inputs of n_tokens rows (bytes; sc: [n_tokens][2] factors) and the
+// product (tile counts and steps are filled in here).
+namespace gk {
+struct WPlanes;
+}
+namespace tk {
+struct ProjGemmArgs;
+}
+hipError_t launch_weight_range(const gk::WPlanes& w, int ggml_type, int rows, int cols, int* rexp, hipStream_t st);
+size_t proj_gemm_input_bytes(int n_tokens, int cols);
+hipError_t launch_tok_split(const float* x, long long x_pitch, int cols, const float* norm_w, float eps, float* sc,
+                            int n_tokens, void* xs, hipStream_t st);
+hipError_t launch_proj_gemm(tk::ProjGemmArgs a, int first_type, int second_type, hipStream_t st);
 // The Q8_1 input of n_tokens rows for the int8 formats (tk::tok_q8_kernel): the single-token
 // kernel's staged norm and quantiser, written in the B-operand layout (q8b: cols/32 * 64
-// uint4, q8d and q8s: cols/32 * kTokBatch floats), kTokBatch slots (zeros past n_tokens); with
+// uint4, q8d and q8s: cols/32 * kTokBatch floats) per group of kTokBatch slots (zeros past n_tokens); with
 // sc, also launch_tok_prep's per-token factors.
 hipError_t launch_tok_q8(const float* x, long long x_pitch, int cols, const float* norm_w, float eps,
                          int n_tokens, void* q8b, float* q8d, float* q8s, float* sc, hipStream_t stream);

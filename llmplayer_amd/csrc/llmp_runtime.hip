@@ -5,7 +5,7 @@
 #include "llmp_internal.h"
 #include "prefill_kernels.h"
 #include "gemv_kernels.h"
-#include "proj_tok_kernels.h"
+#include "proj_gemm_kernels.h"
 
 #include <algorithm>
 #include <cmath>
@@ -16,6 +16,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -48,6 +49,8 @@ struct DevWeight {
     int rows = 0, cols = 0;
     void* mem = nullptr;
     gk::WPlanes planes{};
+    int* rexp = nullptr;   // matrices: [rows] exponents of the many-token projections (in mem),
+    bool rexp_set = false; // filled by the first of them
     // The token-batched projections split fp32 and bf16 weights into fp16 parts: false when
     // some weight reaches fp16's largest magnitude, 65504, or for a type proj_tok_supported
     // rejects (llmp_attn_block_batch then runs the tokens one by one, on the fp32 single-token
@@ -105,6 +108,17 @@ struct KvHandle {
     size_t blk_floats = 0;
     void* blkb_buf = nullptr;        // token-batched block scratch (llmp_attn_block_batch)
     size_t blkb_bytes = 0;
+    // The scratch and the attention workspaces of passes of more than kTokBatch tokens, grown on
+    // demand at least twofold.  They are apart from the ones above, and outgrown ones are kept
+    // until the handle goes, so that no graph captured earlier refers to freed memory.
+    void* many_buf = nullptr;
+    size_t many_bytes = 0;
+    void* many_ws = nullptr;
+    size_t many_ws_bytes = 0;
+    float* many_part = nullptr;
+    size_t many_part_bytes = 0;
+    bool keep_outgrown = false;
+    std::vector<void*> outgrown;
     size_t part_slots = 0;    // (split, query head) slots the workspace holds
     bool prof_on = false;
     std::vector<ProfPair> prof_pending[LLMP_PROF_KINDS];
@@ -216,6 +230,10 @@ void free_handle(KvHandle* kv) {
     }
     if (kv->blk_buf) (void)hipFree(kv->blk_buf);
     if (kv->blkb_buf) (void)hipFree(kv->blkb_buf);
+    if (kv->many_buf) (void)hipFree(kv->many_buf);
+    if (kv->many_ws) (void)hipFree(kv->many_ws);
+    if (kv->many_part) (void)hipFree(kv->many_part);
+    for (void* p : kv->outgrown) (void)hipFree(p);
     if (kv->part_o) (void)hipFree(kv->part_o);
     if (kv->part_ml) (void)hipFree(kv->part_ml);
     if (kv->done) (void)hipFree(kv->done);
@@ -1107,27 +1125,38 @@ int llmp_layer_norm_mode(uint64_t handle, int layer, int mode) {
 }
 
 // ---- attention block: projections around the attention core ------------------------------
-// Byte offsets of the token-batched block scratch: q, k, v, the attention output and the
-// output projection of kTokBatch tokens (each region 256-byte aligned).
+// Byte offsets of the token-batched block scratch for passes of `tokens` tokens: q, k, v, the
+// attention output and the output projection, the per-token factors, and the staged inputs of the
+// projections (each region 256-byte aligned; the output projection only with a post-norm, the
+// Q8_1 staging only in that mode).
 struct BatchLayout {
-    size_t q, k, v, attn, o, sc, q8b, q8d, q8s, total;
+    size_t q, k, v, attn, o, sc, q8b, q8d, q8s, xs, total;
 };
-static BatchLayout batch_layout(const KvHandle* kv, int qd, int kvd) {
+// Tokens from which the projections run as tiled products (proj_gemm_kernels.h): the whole call at
+// the 24/8/128 shape with Q4_K_M weights takes 130 us for 95 tokens in groups of 16 and about 1.15 us
+// more per token; tiled 178 us at 96 tokens and 180 at 200.
+constexpr int kGemmTokens = 136;
+// Tokens of one pass through the projections and the attention: bounds the scratch (about 120 MB
+// at the 24/8/128 shape) at no cost, since a pass this long fills the chip many times over.
+constexpr int kPassTokens = 2048;
+static BatchLayout batch_layout(const KvHandle* kv, int qd, int kvd, int tokens, bool post, bool q8) {
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    const int dim = kv->blk_dim;
+    const int dim = kv->blk_dim, wide = dim > qd ? dim : qd;
+    const size_t groups = ((size_t)tokens + kTokBatch - 1) / kTokBatch, rows = groups * kTokBatch;
     BatchLayout L;
     L.q = 0;
-    L.k = L.q + al((size_t)kTokBatch * qd * sizeof(float));
-    L.v = L.k + al((size_t)kTokBatch * kvd * sizeof(float));
-    L.attn = L.v + al((size_t)kTokBatch * kvd * sizeof(float));
-    L.o = L.attn + al((size_t)kTokBatch * qd * sizeof(float));
-    L.sc = L.o + al((size_t)kTokBatch * dim * sizeof(float));
+    L.k = L.q + al(rows * qd * sizeof(float));
+    L.v = L.k + al(rows * kvd * sizeof(float));
+    L.attn = L.v + al(rows * kvd * sizeof(float));
+    L.o = L.attn + al(rows * qd * sizeof(float));
+    L.sc = L.o + (post ? al(rows * dim * sizeof(float)) : 0);
     // the Q8_1 staging of the widest projection input (dim for Q/K/V, q_dim for Wo)
-    const size_t groups = (size_t)(dim > qd ? dim : qd) / 32;
-    L.q8b = L.sc + al((size_t)kTokBatch * 2 * sizeof(float));
-    L.q8d = L.q8b + al(groups * 64 * 16);
-    L.q8s = L.q8d + al(groups * kTokBatch * sizeof(float));
-    L.total = L.q8s + al(groups * kTokBatch * sizeof(float));
+    const size_t blocks = q8 ? (size_t)wide / 32 : 0;
+    L.q8b = L.sc + al(rows * 2 * sizeof(float));
+    L.q8d = L.q8b + al(groups * blocks * 64 * 16);
+    L.q8s = L.q8d + al(groups * blocks * kTokBatch * sizeof(float));
+    L.xs = L.q8s + al(groups * blocks * kTokBatch * sizeof(float));
+    L.total = L.xs + (!q8 && tokens >= kGemmTokens ? al(proj_gemm_input_bytes(tokens, wide)) : 0);
     return L;
 }
 
@@ -1207,7 +1236,8 @@ int llmp_layer_weight(uint64_t handle, int layer, int slot, int ggml_type, int r
     const int np = repack_weight(ggml_type, rows, cols, static_cast<const uint8_t*>(data), packed, off, pitch);
     if (np == 0)
         return fail(LLMP_ERR_UNSUPPORTED, "llmp_layer_weight: %d columns for GGML type %d", cols, ggml_type);
-    hipError_t e = hipMalloc(&w.mem, packed.size());
+    const size_t rexp_off = KvHandle::pad256(packed.size());
+    hipError_t e = hipMalloc(&w.mem, vec ? packed.size() : rexp_off + (size_t)rows * sizeof(int));
     if (e == hipErrorOutOfMemory)
         return fail(LLMP_ERR_OUT_OF_MEMORY, "llmp_layer_weight: %zu bytes", packed.size());
     LLMP_HIP_CHECK(e, "hipMalloc(weight)");
@@ -1235,6 +1265,7 @@ int llmp_layer_weight(uint64_t handle, int layer, int slot, int ggml_type, int r
         w.planes.p[i] = static_cast<const unsigned char*>(w.mem) + off[i];
         w.planes.pitch[i] = (long long)pitch[i];
     }
+    if (!vec) w.rexp = reinterpret_cast<int*>(static_cast<char*>(w.mem) + rexp_off);
     // Block scratch: q | k | v, the attention output and the Wo output (kept per handle).
     const size_t need = (size_t)(qd + 2 * kvd) + (size_t)qd + (size_t)dim + 64;
     if (need > kv->blk_floats) {
@@ -1247,7 +1278,7 @@ int llmp_layer_weight(uint64_t handle, int layer, int slot, int ggml_type, int r
     }
     // Token-batched block scratch: q, k, v, the attention output and the output projection of
     // 16 tokens.
-    const size_t needb = batch_layout(kv, qd, kvd).total;
+    const size_t needb = batch_layout(kv, qd, kvd, kTokBatch, true, true).total;
     if (needb > kv->blkb_bytes) {
         LLMP_HIP_CHECK(hipDeviceSynchronize(), "hipDeviceSynchronize");
         if (kv->blkb_buf) (void)hipFree(kv->blkb_buf);
@@ -1393,14 +1424,15 @@ static int enqueue_prefill(KvHandle* kv, int layer, int src_layer, int pos0, int
                            bool in_f32, uint64_t q, uint64_t k, uint64_t v, uint64_t gate,
                            uint64_t out, uint64_t stream, bool use_static);
 
+static int batch_pass(KvHandle* kv, int layer, int pos0, int K, float* xc, uint64_t stream);
+
 // The attention half of n_tokens tokens at positions pos0 .. pos0+n_tokens-1 over the rows
 // x[t][dim] (LLMEngine.forwardBatch's per-token forwards, LLMEngine.java:1019-1033, with the
-// projections batched as speculative-decoding.md:120-140 plans): per group of up to kTokBatch
-// tokens, the Q/K/V projections of all of them on the matrix cores (each weight row read once),
-// the multi-token attention on fp32 projections (the rows appended exactly as the single-token
-// decode appends them), the output projection with its residual epilogue, and the post-norm.
-// In the Q8_1 input mode the tokens run one llmp_attn_block call each (that contract's int8 dot
-// products have no batched kernel).
+// projections batched as speculative-decoding.md:120-140 plans): per pass of up to kPassTokens
+// tokens, the Q/K/V projections on the matrix cores (groups of 16 tokens in one launch, or the
+// tiled products from kGemmTokens on), the multi-token attention on fp32 projections (the rows
+// appended exactly as the single-token decode appends them), the output projection with its
+// residual epilogue, and the post-norm.
 int llmp_attn_block_batch(uint64_t handle, int layer, int pos0, int n_tokens, uint64_t x,
                           uint64_t stream) {
     if (int rc = ensure_init()) return rc;
@@ -1423,7 +1455,6 @@ int llmp_attn_block_batch(uint64_t handle, int layer, int pos0, int n_tokens, ui
     const bool w_ok = W[LLMP_W_O].tok_ok && (merged ? W[LLMP_W_QKV].tok_ok
                                                      : W[LLMP_W_Q].tok_ok && W[LLMP_W_K].tok_ok &&
                                                            W[LLMP_W_V].tok_ok);
-    const bool q8 = kv->blk_input == LLMP_INPUT_Q8_1;
     if (prefill_tile_keys(D) <= 0 || !w_ok) {
         // a head size with decode kernels only, fp32 / bf16 weights beyond fp16's range, or a
         // type without a token-batched kernel
@@ -1440,10 +1471,83 @@ int llmp_attn_block_batch(uint64_t handle, int layer, int pos0, int n_tokens, ui
     }
     if (!proj_tok_supported(W[LLMP_W_O].type))
         return fail(LLMP_ERR_UNSUPPORTED, "llmp_attn_block_batch: GGML type %d", W[LLMP_W_O].type);
-    const BatchLayout L = batch_layout(kv, qd, kvd);
-    if (!kv->blkb_buf || L.total > kv->blkb_bytes)
+    // Scratch for passes of several groups of tokens.  Under capture nothing can be allocated: the
+    // passes are then as long as the scratch allows (one group at least, from llmp_layer_weight).
+    hipStream_t st = pick_stream(stream);
+    int pass = n_tokens < kPassTokens ? n_tokens : kPassTokens;
+    if (!kv->blkb_buf || batch_layout(kv, qd, kvd, kTokBatch, true, true).total > kv->blkb_bytes)
         return fail(LLMP_ERR_INVALID_ARG, "llmp_attn_block_batch: layer %d weights not uploaded", layer);
-    char* base = static_cast<char*>(kv->blkb_buf);
+    const size_t need = pass <= kTokBatch ? 0
+                        : batch_layout(kv, qd, kvd, pass, W[LLMP_W_POST_ATTN_NORM].mem != nullptr,
+                                       kv->blk_input == LLMP_INPUT_Q8_1).total;
+    if (need > kv->many_bytes) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        LLMP_HIP_CHECK(hipStreamIsCapturing(st, &cap), "hipStreamIsCapturing");
+        const size_t size = std::max(need, 2 * kv->many_bytes);
+        void* mem = nullptr;
+        if (cap == hipStreamCaptureStatusNone && hipMalloc(&mem, size) == hipSuccess) {
+            if (kv->many_buf) kv->outgrown.push_back(kv->many_buf);
+            kv->many_buf = mem;
+            kv->many_bytes = size;
+        } else {
+            if (cap == hipStreamCaptureStatusNone) (void)hipGetLastError();   // too little memory left
+            pass = kTokBatch;
+        }
+    }
+    for (int t0 = 0; t0 < n_tokens; t0 += pass)
+        if (int rc = batch_pass(kv, layer, pos0 + t0, n_tokens - t0 < pass ? n_tokens - t0 : pass,
+                                reinterpret_cast<float*>(x) + (size_t)t0 * dim, stream))
+            return rc;
+    return LLMP_OK;
+}
+
+// The row exponents of a layer's matrices, computed by its first call of many tokens and complete
+// when this returns, so that any stream may read them.  Under capture nothing can be waited for:
+// *gemm becomes false where some are missing (the groups of 16 need none).
+static int row_exponents(DevWeight* W, bool merged, hipStream_t st, bool* gemm) {
+    bool launched = false;
+    for (int slot = LLMP_W_Q; slot <= LLMP_W_O; ++slot) {
+        DevWeight& w = W[slot];
+        const bool used = slot == LLMP_W_O || (slot == LLMP_W_QKV) == merged;
+        if (!used || w.rexp_set) continue;
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        LLMP_HIP_CHECK(hipStreamIsCapturing(st, &cap), "hipStreamIsCapturing");
+        if (cap != hipStreamCaptureStatusNone) {
+            *gemm = false;
+            return LLMP_OK;
+        }
+        LLMP_HIP_CHECK(launch_weight_range(w.planes, w.type, w.rows, w.cols, w.rexp, st), "weight range launch");
+        launched = true;
+    }
+    if (launched) {
+        LLMP_HIP_CHECK(hipStreamSynchronize(st), "hipStreamSynchronize");
+        for (int slot = LLMP_W_Q; slot <= LLMP_W_O; ++slot)
+            if (slot == LLMP_W_O || (slot == LLMP_W_QKV) == merged) W[slot].rexp_set = true;
+    }
+    return LLMP_OK;
+}
+
+// One pass of llmp_attn_block_batch over K tokens (rows xc), within the handle's scratch.
+static int batch_pass(KvHandle* kv, int layer, int pos0, int K, float* xc, uint64_t stream) {
+    // A group of one token takes the single-token launches, which are faster for it (27 against 49
+    // us at C3), after the others: it attends to their rows.
+    if (K == 1) return enqueue_block(kv, layer, pos0, 0, reinterpret_cast<uint64_t>(xc), 0, stream);
+    if (K % kTokBatch == 1 && (kv->blk_input == LLMP_INPUT_Q8_1 || K < kGemmTokens)) {
+        if (int rc = batch_pass(kv, layer, pos0, K - 1, xc, stream)) return rc;
+        return batch_pass(kv, layer, pos0 + K - 1, 1, xc + (size_t)(K - 1) * kv->blk_dim, stream);
+    }
+    const LayerCfg& c = kv->layers[(size_t)layer];
+    const DevWeight* W = c.w;
+    const bool merged = W[LLMP_W_QKV].mem != nullptr;
+    const int D = kv->head_dim, qd = c.n_heads * D, kvd = kv->n_kv_heads * D, dim = kv->blk_dim;
+    const bool q8 = kv->blk_input == LLMP_INPUT_Q8_1;
+    hipStream_t st = pick_stream(stream);
+    bool gemm = !q8 && K >= kGemmTokens;
+    if (gemm)
+        if (int rc = row_exponents(kv->layers[(size_t)layer].w, merged, st, &gemm)) return rc;
+    const BatchLayout L = batch_layout(kv, qd, kvd, K, W[LLMP_W_POST_ATTN_NORM].mem != nullptr, q8);
+    const bool many = K > kTokBatch;
+    char* base = static_cast<char*>(many ? kv->many_buf : kv->blkb_buf);
     float* qb = reinterpret_cast<float*>(base + L.q);
     float* kb = reinterpret_cast<float*>(base + L.k);
     float* vb = reinterpret_cast<float*>(base + L.v);
@@ -1453,21 +1557,23 @@ int llmp_attn_block_batch(uint64_t handle, int layer, int pos0, int n_tokens, ui
     void* q8b = base + L.q8b;
     float* q8d = reinterpret_cast<float*>(base + L.q8d);
     float* q8s = reinterpret_cast<float*>(base + L.q8s);
-    hipStream_t st = pick_stream(stream);
+    void* xs = base + L.xs;
     auto vecp = [&](int slot) -> const float* { return static_cast<const float*>(W[slot].mem); };
 
     // Q/K/V segments: outputs q [K][qd], k [K][kvd], v [K][kvd].
     tk::TokSeg segs[3];
+    tk::GemmSeg gsegs[3];
     int types[3];
     const int seg_rows[3] = {qd, kvd, kvd}, seg_off[3] = {0, qd, qd + kvd};
     const int bias_slot[3] = {LLMP_W_Q_BIAS, LLMP_W_K_BIAS, LLMP_W_V_BIAS};
     float* seg_out[3] = {qb, kb, vb};
     for (int i = 0; i < 3; ++i) {
         const DevWeight& dw = merged ? W[LLMP_W_QKV] : W[LLMP_W_Q + i];
+        const int off = merged ? seg_off[i] : 0;   // rows off.. of the merged matrix
         segs[i].w = dw.planes;
         if (merged)
             for (int p = 0; p < 4; ++p)
-                if (dw.planes.p[p]) segs[i].w.p[p] = dw.planes.p[p] + (long long)seg_off[i] * dw.planes.pitch[p];
+                if (dw.planes.p[p]) segs[i].w.p[p] = dw.planes.p[p] + (long long)off * dw.planes.pitch[p];
         segs[i].rows = seg_rows[i];
         segs[i].out_off = seg_off[i];
         segs[i].fmt = 0;
@@ -1475,6 +1581,7 @@ int llmp_attn_block_batch(uint64_t handle, int layer, int pos0, int n_tokens, ui
         segs[i].out = seg_out[i];
         segs[i].out_pitch = seg_rows[i];
         types[i] = dw.type;
+        gsegs[i] = {segs[i].w, seg_rows[i], 0, 0, dw.rexp + off, segs[i].bias, seg_out[i], seg_rows[i]};
     }
     // One launch when the three share a type or form a supported pair (the Q4_K_M mix);
     // otherwise one per run of segments of one type.
@@ -1486,32 +1593,45 @@ int llmp_attn_block_batch(uint64_t handle, int layer, int pos0, int n_tokens, ui
         }
     if (t2 >= 0 && !proj_tok_pair_supported(t1, t2) && proj_tok_pair_supported(t2, t1)) std::swap(t1, t2);
     const bool paired = t2 >= 0 && proj_tok_pair_supported(t1, t2);
-    float* xp = reinterpret_cast<float*>(x);
-    for (int t0 = 0; t0 < n_tokens; t0 += kTokBatch) {
-        const int K = n_tokens - t0 < kTokBatch ? n_tokens - t0 : kTokBatch;
-        float* xc = xp + (size_t)t0 * dim;
-        if (K == 1) {   // one token: the single-token launches are faster (27 against 49 µs at C3)
-            if (int rc = enqueue_block(kv, layer, pos0 + t0, 0, reinterpret_cast<uint64_t>(xc), 0, stream))
-                return rc;
-            continue;
-        }
-        // 1-2. The tokens' pre-norm factors and input range exponents, then the Q/K/V
-        //      projections of the normalised inputs.
-        // In the Q8_1 mode the tokens' quantised inputs come with the same factors.
-        if (q8)
-            LLMP_HIP_CHECK(launch_tok_q8(xc, dim, dim, vecp(LLMP_W_ATTN_NORM), c.eps, K, q8b, q8d, q8s, sc, st),
-                           "batched block Q8_1 input launch");
-        else
-            LLMP_HIP_CHECK(launch_tok_prep(xc, dim, dim, vecp(LLMP_W_ATTN_NORM), c.eps, sc, K, st),
-                           "batched block input prep launch");
-        if (paired || t2 == -1) {
-            tk::ProjTokArgs g{};
-            for (int k = 0; k < 3; ++k) {
-                g.seg[k] = segs[k];
-                g.seg[k].fmt = types[k] == t1 ? 0 : 1;
+    // 1-2. The tokens' pre-norm factors and input exponents (and their quantised or split inputs),
+    //      then the Q/K/V projections of the normalised inputs.
+    if (gemm)
+        LLMP_HIP_CHECK(launch_tok_split(xc, dim, dim, vecp(LLMP_W_ATTN_NORM), c.eps, sc, K, xs, st),
+                       "batched block input split launch");
+    else if (q8)
+        LLMP_HIP_CHECK(launch_tok_q8(xc, dim, dim, vecp(LLMP_W_ATTN_NORM), c.eps, K, q8b, q8d, q8s, sc, st),
+                       "batched block Q8_1 input launch");
+    else
+        LLMP_HIP_CHECK(launch_tok_prep(xc, dim, dim, vecp(LLMP_W_ATTN_NORM), c.eps, sc, K, st),
+                       "batched block input prep launch");
+    for (int i = 0; i < 3;) {
+        int n = 3;
+        if (!paired && t2 != -1)
+            for (n = 1; i + n < 3 && types[i + n] == types[i];) ++n;
+        const int first = paired ? t1 : types[i], second = paired ? t2 : -1;
+        if (gemm) {
+            tk::ProjGemmArgs g{};
+            for (int k = 0; k < n; ++k) {
+                g.seg[k] = gsegs[i + k];
+                g.seg[k].fmt = types[i + k] == first ? 0 : 1;
             }
-            g.nseg = 3;
-            g.rows_total = qd + 2 * kvd;
+            g.nseg = n;
+            g.cols = dim;
+            g.K = K;
+            g.xs = static_cast<const uint4*>(xs);
+            g.tok_sc = sc;
+            LLMP_HIP_CHECK(launch_proj_gemm(g, first, second, st), "batched block Q/K/V projection launch");
+        } else {
+            tk::ProjTokArgs g{};
+            int off = 0;
+            for (int k = 0; k < n; ++k) {
+                g.seg[k] = segs[i + k];
+                g.seg[k].fmt = types[i + k] == first ? 0 : 1;
+                g.seg[k].out_off = off;
+                off += segs[i + k].rows;
+            }
+            g.nseg = n;
+            g.rows_total = off;
             g.cols = dim;
             g.K = K;
             g.x = xc;
@@ -1522,42 +1642,47 @@ int llmp_attn_block_batch(uint64_t handle, int layer, int pos0, int n_tokens, ui
             g.q8b = static_cast<const uint4*>(q8b);
             g.q8d = q8d;
             g.q8s = q8s;
-            LLMP_HIP_CHECK(launch_proj_tok(g, t1, paired ? t2 : -1, q8, st), "batched block Q/K/V projection launch");
-        } else {
-            for (int i = 0; i < 3;) {
-                int n = 1;
-                while (i + n < 3 && types[i + n] == types[i]) ++n;
-                tk::ProjTokArgs g{};
-                int off = 0;
-                for (int k = 0; k < n; ++k) {
-                    g.seg[k] = segs[i + k];
-                    g.seg[k].out_off = off;
-                    off += segs[i + k].rows;
-                }
-                g.nseg = n;
-                g.rows_total = off;
-                g.cols = dim;
-                g.K = K;
-                g.x = xc;
-                g.x_pitch = dim;
-                g.norm_w = vecp(LLMP_W_ATTN_NORM);
-                g.tok_sc = sc;
-                g.eps = c.eps;
-                g.q8b = static_cast<const uint4*>(q8b);
-                g.q8d = q8d;
-                g.q8s = q8s;
-                LLMP_HIP_CHECK(launch_proj_tok(g, types[i], -1, q8, st), "batched block Q/K/V projection launch");
-                i += n;
-            }
+            LLMP_HIP_CHECK(launch_proj_tok(g, first, second, q8, st), "batched block Q/K/V projection launch");
         }
-        // 3-5. Attention of the K tokens (QK-norm, RoPE, exact appends, causal over the cache).
-        if (int rc = enqueue_prefill(kv, layer, -1, pos0 + t0, K, true, reinterpret_cast<uint64_t>(qb),
-                                     reinterpret_cast<uint64_t>(kb), reinterpret_cast<uint64_t>(vb), 0,
-                                     reinterpret_cast<uint64_t>(attn), stream, false))
-            return rc;
-        // 6. Output projection (+ bias), post-norm, residual scale and residual add.
+        i += n;
+    }
+    // 3-5. Attention of the K tokens (QK-norm, RoPE, exact appends, causal over the cache).
+    auto swap_workspaces = [&] {
+        if (!many) return;
+        std::swap(kv->prefill_ws, kv->many_ws);
+        std::swap(kv->prefill_ws_bytes, kv->many_ws_bytes);
+        std::swap(kv->prefill_part, kv->many_part);
+        std::swap(kv->prefill_part_bytes, kv->many_part_bytes);
+        kv->keep_outgrown = !kv->keep_outgrown;
+    };
+    swap_workspaces();
+    const int rc = enqueue_prefill(kv, layer, -1, pos0, K, true, reinterpret_cast<uint64_t>(qb),
+                                   reinterpret_cast<uint64_t>(kb), reinterpret_cast<uint64_t>(vb), 0,
+                                   reinterpret_cast<uint64_t>(attn), stream, false);
+    swap_workspaces();
+    if (rc) return rc;
+    // 6. Output projection (+ bias), post-norm, residual scale and residual add.
+    const float* post = vecp(LLMP_W_POST_ATTN_NORM);
+    const DevWeight& wo = W[LLMP_W_O];
+    if (gemm) {
+        LLMP_HIP_CHECK(launch_tok_split(attn, qd, qd, nullptr, 0.0f, sc, K, xs, st),
+                       "batched block attention-output split launch");
+        tk::ProjGemmArgs g{};
+        g.seg[0] = {wo.planes, dim, 0, 0, wo.rexp, vecp(LLMP_W_O_BIAS), ob, dim};
+        g.nseg = 1;
+        g.cols = qd;
+        g.K = K;
+        g.xs = static_cast<const uint4*>(xs);
+        g.tok_sc = sc;
+        if (!post) {
+            g.resid = xc;
+            g.resid_pitch = dim;
+            g.rscale = kv->blk_rscale;
+        }
+        LLMP_HIP_CHECK(launch_proj_gemm(g, wo.type, -1, st), "batched block output projection launch");
+    } else {
         tk::ProjTokArgs g{};
-        g.seg[0].w = W[LLMP_W_O].planes;
+        g.seg[0].w = wo.planes;
         g.seg[0].rows = dim;
         g.seg[0].bias = vecp(LLMP_W_O_BIAS);
         g.nseg = 1;
@@ -1568,7 +1693,7 @@ int llmp_attn_block_batch(uint64_t handle, int layer, int pos0, int n_tokens, ui
         g.x_pitch = qd;
         g.in_range = kv->range(layer);   // |attention output| <= the largest stored |V|
         g.in_range_n = kv->n_kv_heads;
-        const bool wo_q8 = q8 && proj_tok_q8_routed(W[LLMP_W_O].type);
+        const bool wo_q8 = q8 && proj_tok_q8_routed(wo.type);
         if (wo_q8) {   // the attention output quantised, as the single-token kernel does
             LLMP_HIP_CHECK(launch_tok_q8(attn, qd, qd, nullptr, 0.0f, K, q8b, q8d, q8s, nullptr, st),
                            "batched block Q8_1 attention-output launch");
@@ -1576,20 +1701,19 @@ int llmp_attn_block_batch(uint64_t handle, int layer, int pos0, int n_tokens, ui
             g.q8d = q8d;
             g.q8s = q8s;
         }
-        const float* post = vecp(LLMP_W_POST_ATTN_NORM);
         if (post) {
             g.seg[0].out = ob;
             g.seg[0].out_pitch = dim;
-            LLMP_HIP_CHECK(launch_proj_tok(g, W[LLMP_W_O].type, -1, wo_q8, st), "batched block output projection launch");
-            LLMP_HIP_CHECK(launch_post_norm_residual(ob, post, c.eps, kv->blk_rscale, xc, dim, K, st),
-                           "batched block post-norm launch");
         } else {
             g.resid = xc;
             g.resid_pitch = dim;
             g.rscale = kv->blk_rscale;
-            LLMP_HIP_CHECK(launch_proj_tok(g, W[LLMP_W_O].type, -1, wo_q8, st), "batched block output projection launch");
         }
+        LLMP_HIP_CHECK(launch_proj_tok(g, wo.type, -1, wo_q8, st), "batched block output projection launch");
     }
+    if (post)
+        LLMP_HIP_CHECK(launch_post_norm_residual(ob, post, c.eps, kv->blk_rscale, xc, dim, K, st),
+                       "batched block post-norm launch");
     return LLMP_OK;
 }
 
@@ -1812,35 +1936,31 @@ static int enqueue_prefill(KvHandle* kv, int layer, int src_layer, int pos0, int
         if (!ws) return fail(LLMP_ERR_NOT_INIT, "llmp_attn_prefill_f32_static: no scratch address");
         a.part_o = reinterpret_cast<float*>(static_cast<char*>(ws) + ws_bytes);
     } else {
-        if (ws_bytes > kv->prefill_ws_bytes) {
-            if (kv->prefill_ws) {
+        // A growth frees the smaller workspace behind the stream's work on it, or keeps it
+        // (KvHandle::keep_outgrown).
+        auto grow = [&](auto*& buf, size_t& have, size_t need, const char* what) -> int {
+            if (need <= have) return LLMP_OK;
+            void* old = buf;
+            if (old && !kv->keep_outgrown) {
                 LLMP_HIP_CHECK(hipStreamSynchronize(st), "hipStreamSynchronize");
-                (void)hipFree(kv->prefill_ws);
-                kv->prefill_ws = nullptr;
-                kv->prefill_ws_bytes = 0;
+                (void)hipFree(old);
+                buf = nullptr;
+                have = 0;
             }
-            hipError_t e = hipMalloc(&kv->prefill_ws, ws_bytes);
-            if (e == hipErrorOutOfMemory)
-                return fail(LLMP_ERR_OUT_OF_MEMORY, "llmp_attn_prefill: %zu-byte tile workspace", ws_bytes);
+            if (kv->keep_outgrown) need = std::max(need, 2 * have);
+            void* mem = nullptr;
+            hipError_t e = hipMalloc(&mem, need);
+            if (e == hipErrorOutOfMemory) return fail(LLMP_ERR_OUT_OF_MEMORY, "llmp_attn_prefill: %zu-byte %s", need, what);
             LLMP_HIP_CHECK(e, "hipMalloc(prefill workspace)");
-            kv->prefill_ws_bytes = ws_bytes;
-        }
+            if (old && kv->keep_outgrown) kv->outgrown.push_back(old);
+            buf = static_cast<std::remove_reference_t<decltype(buf)>>(mem);
+            have = need;
+            return LLMP_OK;
+        };
+        if (int rc = grow(kv->prefill_ws, kv->prefill_ws_bytes, ws_bytes, "tile workspace")) return rc;
         ws = kv->prefill_ws;
         // Key splits (chunks whose query blocks leave CUs idle) and their partials buffer.
-        if (part_bytes > kv->prefill_part_bytes) {
-            if (kv->prefill_part) {
-                LLMP_HIP_CHECK(hipStreamSynchronize(st), "hipStreamSynchronize");
-                (void)hipFree(kv->prefill_part);
-                kv->prefill_part = nullptr;
-                kv->prefill_part_bytes = 0;
-            }
-            hipError_t e = hipMalloc(&kv->prefill_part, part_bytes);
-            if (e == hipErrorOutOfMemory)
-                return fail(LLMP_ERR_OUT_OF_MEMORY, "llmp_attn_prefill: %zu-byte split workspace",
-                            part_bytes);
-            LLMP_HIP_CHECK(e, "hipMalloc(prefill partials)");
-            kv->prefill_part_bytes = part_bytes;
-        }
+        if (int rc = grow(kv->prefill_part, kv->prefill_part_bytes, part_bytes, "split workspace")) return rc;
         a.part_o = kv->prefill_part;
     }
     if (ksplit > 1) a.part_ml = a.part_o + (size_t)ksplit * n_tokens * c.n_heads * D;

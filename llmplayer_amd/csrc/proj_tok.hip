@@ -9,11 +9,12 @@ namespace {
 
 template <class F1, class F2>
 hipError_t launch_ff(const tk::ProjTokArgs& a, hipStream_t st) {
+    const dim3 grid(a.rows_total / 16, (a.K + tk::kTok - 1) / tk::kTok);
     if (a.norm_w != nullptr)
-        hipLaunchKernelGGL((tk::proj_tok_kernel<F1, F2, true>), dim3(a.rows_total / 16), dim3(tk::kThreads),
+        hipLaunchKernelGGL((tk::proj_tok_kernel<F1, F2, true>), grid, dim3(tk::kThreads),
                            (size_t)a.cols * sizeof(float), st, a);
     else
-        hipLaunchKernelGGL((tk::proj_tok_kernel<F1, F2, false>), dim3(a.rows_total / 16), dim3(tk::kThreads),
+        hipLaunchKernelGGL((tk::proj_tok_kernel<F1, F2, false>), grid, dim3(tk::kThreads),
                            0, st, a);
     return hipGetLastError();
 }
@@ -23,7 +24,7 @@ hipError_t launch_ff(const tk::ProjTokArgs& a, hipStream_t st) {
 hipError_t launch_tok_prep(const float* x, long long x_pitch, int cols, const float* norm_w, float eps,
                            float* sc, int n_tokens, hipStream_t st) {
     if (x == nullptr || sc == nullptr || cols <= 0 || (cols & 3) || (x_pitch & 3) || n_tokens < 1 ||
-        n_tokens > tk::kTok || (reinterpret_cast<uintptr_t>(x) & 15) || (reinterpret_cast<uintptr_t>(norm_w) & 15))
+        (reinterpret_cast<uintptr_t>(x) & 15) || (reinterpret_cast<uintptr_t>(norm_w) & 15))
         return hipErrorInvalidValue;
     hipLaunchKernelGGL(tk::tok_prep_kernel<tk::kPrepThreads>, dim3(n_tokens), dim3(tk::kPrepThreads), 0, st, x, x_pitch,
                        cols, norm_w, eps, sc);
@@ -33,12 +34,13 @@ hipError_t launch_tok_prep(const float* x, long long x_pitch, int cols, const fl
 hipError_t launch_tok_q8(const float* x, long long x_pitch, int cols, const float* norm_w, float eps,
                          int n_tokens, void* q8b, float* q8d, float* q8s, float* sc, hipStream_t st) {
     if (x == nullptr || q8b == nullptr || q8d == nullptr || q8s == nullptr || cols <= 0 || (cols & 31) ||
-        cols > gk::kMaxGemvCols || (x_pitch & 3) || n_tokens < 1 || n_tokens > tk::kTok ||
+        cols > gk::kMaxGemvCols || (x_pitch & 3) || n_tokens < 1 ||
         (reinterpret_cast<uintptr_t>(x) & 15) || (reinterpret_cast<uintptr_t>(norm_w) & 15) ||
         (reinterpret_cast<uintptr_t>(q8b) & 15))
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(tk::tok_q8_kernel<tk::kPrepThreads>, dim3(tk::kTok), dim3(tk::kPrepThreads), (size_t)cols,
-                       st, x, x_pitch, cols, norm_w, eps, n_tokens, static_cast<uint4*>(q8b), q8d, q8s, sc);
+    hipLaunchKernelGGL(tk::tok_q8_kernel<tk::kPrepThreads>, dim3(tk::kTok, (n_tokens + tk::kTok - 1) / tk::kTok),
+                       dim3(tk::kPrepThreads), (size_t)cols, st, x, x_pitch, cols, norm_w, eps, n_tokens,
+                       static_cast<uint4*>(q8b), q8d, q8s, sc);
     return hipGetLastError();
 }
 
@@ -94,7 +96,7 @@ hipError_t launch_q8(const tk::ProjTokArgs& a, int first_type, int second_type, 
 
 hipError_t launch_proj_tok(const tk::ProjTokArgs& a, int first_type, int second_type, bool q8, hipStream_t st) {
     if ((a.norm_w != nullptr && a.tok_sc == nullptr) || a.cols <= 0 || a.cols % 32 || a.rows_total <= 0 || a.rows_total % 16 || a.K < 1 ||
-        a.K > tk::kTok || a.nseg < 1 || a.nseg > 3 || a.x == nullptr || (a.x_pitch & 3) ||
+        a.nseg < 1 || a.nseg > 3 || a.x == nullptr || (a.x_pitch & 3) ||
         (reinterpret_cast<uintptr_t>(a.x) & 15) || (reinterpret_cast<uintptr_t>(a.norm_w) & 15) ||
         a.cols > gk::kMaxGemvCols)
         return hipErrorInvalidValue;

@@ -76,7 +76,7 @@ struct ProjTokArgs {
     int nseg;
     int rows_total;        // sum of the segments' rows (a multiple of 16)
     int cols;              // a multiple of 32
-    int K;                 // tokens, 1..16
+    int K;                 // tokens: groups of 16 along the grid's y
     const float* x;        // inputs [K][x_pitch] fp32 (16-byte aligned rows)
     long long x_pitch;
     const float* norm_w;   // pre-norm weights [cols] (RMSNorm of each input row), or nullptr
@@ -779,33 +779,44 @@ struct PF32 {
 };
 
 // ---- input range and pre-norm factors -------------------------------------------------------
-// The launch's input range exponent E (ProjTokArgs::tok_sc), uniform over the workgroup.
-__device__ __forceinline__ int input_exp(const ProjTokArgs& a) {
+// A workgroup's group of 16 tokens (grid y): its first token, its tokens and their inputs.
+struct TokGroup {
+    int t0, K;
+    const float* x;
+    const float* tok_sc;
+    const uint4* q8b;
+    const float *q8d, *q8s;
+};
+__device__ __forceinline__ TokGroup tok_group(const ProjTokArgs& a) {
+    const int y = blockIdx.y, t0 = y * kTok, n_grp = a.cols >> 5;
+    return {t0, min(kTok, a.K - t0), a.x + (long long)t0 * a.x_pitch, a.tok_sc == nullptr ? nullptr : a.tok_sc + 2 * t0,
+            a.q8b + (size_t)y * n_grp * 64, a.q8d + (size_t)y * n_grp * kTok, a.q8s + (size_t)y * n_grp * kTok};
+}
+// The group's input range exponent E (ProjTokArgs::tok_sc), uniform over the workgroup.
+__device__ __forceinline__ int input_exp(const ProjTokArgs& a, const TokGroup& tg) {
     int e = 0;
-    if (a.tok_sc != nullptr) {
-        for (int t = 0; t < a.K; ++t) e = max(e, (int)a.tok_sc[2 * t + 1]);
+    if (tg.tok_sc != nullptr) {
+        for (int t = 0; t < tg.K; ++t) e = max(e, (int)tg.tok_sc[2 * t + 1]);
     } else if (a.in_range != nullptr) {
         for (int h = 0; h < a.in_range_n; ++h) e = max(e, a.in_range[2 * h + 1]);
     }
     return __builtin_amdgcn_readfirstlane(e);
 }
 
-// One workgroup per token t: with norm weights w, r = 1/sqrt(sum(x^2)/cols + eps) (the factor
-// of RMSNorm.apply, RMSNorm.java:13-22) and e the range exponent (dk::range_exp_of_bits) of
-// max |x*w| (the values the projection splits); without, r = 1 and e from max |x|.  Writes
-// sc[2t] = r and sc[2t + 1] = e.  x rows and w are 16-byte aligned and cols % 4 == 0
+// Over one row x, by one workgroup (results in thread 0): with norm weights w, r =
+// 1/sqrt(sum(x^2)/cols + eps) (the factor of RMSNorm.apply, RMSNorm.java:13-22) and m the bits of
+// max |x*w| (the values the projection splits); without, r = 1 and m from max |x|.  x rows and w are 16-byte aligned and cols % 4 == 0
 // (launch_tok_prep checks).  One pass: each trip issues all of its float4 loads before any
 // arithmetic, so a row of up to 4·4·NTHR values costs one memory round trip (a loop with one
 // dependent load per trip waited a full round trip per trip: 9.7 µs for 16 rows of 3072).
 constexpr int kPrepThreads = 256;
 constexpr int kPrepUnroll = 4;
 template <int NTHR>
-__global__ __launch_bounds__(NTHR) void tok_prep_kernel(const float* x, long long x_pitch, int cols,
-                                                        const float* w, float eps, float* sc) {
+__device__ __forceinline__ void tok_reduce(const float* x, int cols, const float* w, float eps, float& r, unsigned& m) {
     __shared__ float red[NTHR / 64];
     __shared__ unsigned redm[NTHR / 64];
-    const int tid = threadIdx.x, t = blockIdx.x;
-    const float4* xt = reinterpret_cast<const float4*>(x + (long long)t * x_pitch);
+    const int tid = threadIdx.x;
+    const float4* xt = reinterpret_cast<const float4*>(x);
     const float4* w4 = reinterpret_cast<const float4*>(w);
     const int n4 = cols >> 2;
     const bool norm = w != nullptr;
@@ -842,20 +853,32 @@ __global__ __launch_bounds__(NTHR) void tok_prep_kernel(const float* x, long lon
         redm[tid >> 6] = mb;
     }
     __syncthreads();
+    r = 1.0f;
+    m = redm[0];
     if (tid == 0) {
         float tot = red[0];
-        unsigned m = redm[0];
 #pragma unroll
         for (int k = 1; k < NTHR / 64; ++k) {
             tot = tot + red[k];
             m = max(m, redm[k]);
         }
-        float r = 1.0f;
         if (norm) {
             float q = tot / (float)cols;
             q = q + eps;
             r = 1.0f / (float)__builtin_sqrt((double)q);
         }
+    }
+}
+
+// tok_reduce per token t = blockIdx.x: sc[2t] = r, sc[2t + 1] = the range exponent of m.
+template <int NTHR>
+__global__ __launch_bounds__(NTHR) void tok_prep_kernel(const float* x, long long x_pitch, int cols,
+                                                        const float* w, float eps, float* sc) {
+    const int t = blockIdx.x;
+    float r;
+    unsigned m;
+    tok_reduce<NTHR>(x + (long long)t * x_pitch, cols, w, eps, r, m);
+    if (threadIdx.x == 0) {
         sc[2 * t] = r;
         sc[2 * t + 1] = (float)dk::range_exp_of_bits(m);
     }
@@ -881,6 +904,13 @@ __global__ __launch_bounds__(NTHR) void tok_q8_kernel(const float* x, long long 
     __shared__ unsigned redm[NTHR / 64];
     const int tid = threadIdx.x, t = blockIdx.x, lane = tid & 63;
     const int n4 = cols >> 2, ng = cols >> 5;
+    const int t_base = (int)blockIdx.y * kTok;   // group of 16 tokens
+    n_tokens -= t_base;
+    x += (long long)t_base * x_pitch;
+    q8b += (size_t)blockIdx.y * ng * 64;
+    q8d += (size_t)blockIdx.y * ng * kTok;
+    q8s += (size_t)blockIdx.y * ng * kTok;
+    if (sc != nullptr) sc += 2 * t_base;
     if (t >= n_tokens) {
         for (int i = tid; i < 4 * ng; i += NTHR) q8b[64 * (i >> 2) + 16 * (i & 3) + t] = make_uint4(0u, 0u, 0u, 0u);
         for (int g = tid; g < ng; g += NTHR) {
@@ -973,7 +1003,7 @@ struct ChunkRegs<F, true> {   // the Q8_1 input: the quants as fp16, the block s
 };
 
 template <class F, bool NORM>
-__device__ __forceinline__ void chunk_issue(ChunkRegs<F>& c, const ProjTokArgs& a, const WPlanes& w,
+__device__ __forceinline__ void chunk_issue(ChunkRegs<F>& c, const ProjTokArgs& a, const TokGroup& tg, const WPlanes& w,
                                             int row, int ch, int ngroups, int lane, bool tok_live) {
     const int kq = lane >> 4, t = lane & 15;
     const int g0 = ch * kGroups;
@@ -983,13 +1013,13 @@ __device__ __forceinline__ void chunk_issue(ChunkRegs<F>& c, const ProjTokArgs& 
 #pragma unroll
         for (int gi = 0; gi < kGroups; ++gi) {
             const int g = g0 + min(gi, ng - 1);
-            c.b[gi] = a.q8b[64 * g + lane];
-            c.dx[gi] = a.q8d[16 * g + t];
-            c.sx[gi] = a.q8s[16 * g + t];
+            c.b[gi] = tg.q8b[64 * g + lane];
+            c.dx[gi] = tg.q8d[16 * g + t];
+            c.sx[gi] = tg.q8s[16 * g + t];
         }
     } else {
         // lanes of tokens past K load token K-1's row (no branch between the loads)
-        const float* xt = a.x + (long long)(tok_live ? t : a.K - 1) * a.x_pitch;
+        const float* xt = tg.x + (long long)(tok_live ? t : tg.K - 1) * a.x_pitch;
 #pragma unroll
         for (int gi = 0; gi < kGroups; ++gi) {
             const int col = 32 * (g0 + min(gi, ng - 1)) + 8 * kq;
@@ -1117,15 +1147,15 @@ __device__ __forceinline__ void chunk_consume(const ChunkRegs<F>& c, f32x4_t& ac
 // refill made the wait-count pass merge the two paths, and each chunk then waited for the next
 // chunk's loads.
 template <class F, bool NORM>
-__device__ __forceinline__ void wave_rows(const ProjTokArgs& a, const WPlanes& w, int row, int wave,
+__device__ __forceinline__ void wave_rows(const ProjTokArgs& a, const TokGroup& tg, const WPlanes& w, int row, int wave,
                                           int lane, f32x4_t& acc, float fin, float* tab, float* s_nw) {
     const int ngroups = a.cols >> 5;
     const int nchunks = (ngroups + kGroups - 1) / kGroups;
     const int n = wave < nchunks ? (nchunks - wave + kWaves - 1) / kWaves : 0;
-    const bool tok_live = (lane & 15) < a.K;
+    const bool tok_live = (lane & 15) < tg.K;
     auto chunk = [&](int i) { return wave + min(i, n - 1) * kWaves; };
     ChunkRegs<F> ca, cb;
-    if (n > 0) chunk_issue<F, NORM>(ca, a, w, row, chunk(0), ngroups, lane, tok_live);
+    if (n > 0) chunk_issue<F, NORM>(ca, a, tg, w, row, chunk(0), ngroups, lane, tok_live);
     constexpr int GRID = gk::FmtGrid<F>::BYTES;   // codebook formats: the codebook to LDS
     constexpr bool STAGE_NW = NORM && !IsQ8B<F>::value;   // the Q8_1 input is normalised already
     if constexpr (STAGE_NW || GRID > 0) {
@@ -1147,9 +1177,9 @@ __device__ __forceinline__ void wave_rows(const ProjTokArgs& a, const WPlanes& w
     if (n == 0) return;
     int i = 0;
     for (; i + 1 < n; i += 2) {
-        chunk_issue<F, NORM>(cb, a, w, row, chunk(i + 1), ngroups, lane, tok_live);
+        chunk_issue<F, NORM>(cb, a, tg, w, row, chunk(i + 1), ngroups, lane, tok_live);
         chunk_consume<F, NORM>(ca, acc, fin, tab, s_nw, chunk(i), ngroups, lane);
-        chunk_issue<F, NORM>(ca, a, w, row, chunk(i + 2), ngroups, lane, tok_live);
+        chunk_issue<F, NORM>(ca, a, tg, w, row, chunk(i + 2), ngroups, lane, tok_live);
         chunk_consume<F, NORM>(cb, acc, fin, tab, s_nw, chunk(i + 1), ngroups, lane);
     }
     if (n & 1) chunk_consume<F, NORM>(ca, acc, fin, tab, s_nw, chunk(n - 1), ngroups, lane);
@@ -1172,6 +1202,7 @@ template <class F1, class F2, bool NORM>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(waves_per_eu<F1, F2>())))
 void proj_tok_kernel(ProjTokArgs a) {
     extern __shared__ float s_nw[];   // NORM: the pre-norm weights [cols], times 2^-E
+    const TokGroup tg = tok_group(a);
     __shared__ float s_tab[kWaves][16 * tab_floats<F1, F2>()];
     __shared__ f32x4_t s_red[kWaves][64];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -1181,12 +1212,12 @@ void proj_tok_kernel(ProjTokArgs a) {
     const int row = row0 - sg.out_off + (lane & 15);   // this lane's A row within its segment
     f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
     // The launch's input range factor 2^-E and output factor 2^E (scalar registers).
-    const int E = input_exp(a);
+    const int E = input_exp(a, tg);
     const float fin = __uint_as_float((unsigned)(127 - E) << 23);
     if (std::is_same<F1, F2>::value || sg.fmt == 0)
-        wave_rows<F1, NORM>(a, sg.w, row, wave, lane, acc, fin, s_tab[wave], s_nw);
+        wave_rows<F1, NORM>(a, tg, sg.w, row, wave, lane, acc, fin, s_tab[wave], s_nw);
     else
-        wave_rows<F2, NORM>(a, sg.w, row, wave, lane, acc, fin, s_tab[wave], s_nw);
+        wave_rows<F2, NORM>(a, tg, sg.w, row, wave, lane, acc, fin, s_tab[wave], s_nw);
 
     s_red[wave][lane] = acc;
     __syncthreads();
@@ -1201,19 +1232,19 @@ void proj_tok_kernel(ProjTokArgs a) {
         // rows on the Q8_1 input carry its scales already (no 2^-E, normalised before quantising)
         const bool first = std::is_same<F1, F2>::value || sg.fmt == 0;
         const bool q8_rows = first ? IsQ8B<F1>::value : IsQ8B<F2>::value;
-        if (tt < a.K) {
+        if (tt < tg.K) {
             if (!q8_rows) {
                 v = v * __uint_as_float((unsigned)(127 + E) << 23);   // the inputs were scaled by 2^-E
-                if constexpr (NORM) v = v * a.tok_sc[2 * tt];         // RMSNorm.apply's factor r
+                if constexpr (NORM) v = v * tg.tok_sc[2 * tt];         // RMSNorm.apply's factor r
             }
             const int r = row0 - sg.out_off + rr;
             if (sg.bias != nullptr) v = v + sg.bias[r];
             if (a.resid != nullptr) {
                 if (a.rscale > 0.0f) v = v * a.rscale;
-                float* x = a.resid + (long long)tt * a.resid_pitch + row0 + rr;
+                float* x = a.resid + (long long)(tg.t0 + tt) * a.resid_pitch + row0 + rr;
                 *x = *x + v;
             } else {
-                sg.out[(long long)tt * sg.out_pitch + r] = v;
+                sg.out[(long long)(tg.t0 + tt) * sg.out_pitch + r] = v;
             }
         }
     }

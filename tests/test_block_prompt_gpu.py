@@ -1,0 +1,142 @@
+"""GPU parity of the attention half for a prompt's worth of tokens (llmp_attn_block_batch with the
+tiled projections of proj_gemm_kernels.h, from 136 tokens, and the 16-token groups of one launch
+below) against sequential oracle calls, at the bars of test_block_batch_gpu: every weight format,
+tile edges (rows no multiple of 64, columns no multiple of 128, tokens around a tile of 128),
+mixes in one launch, the epilogues, and inputs and weights far from fp16's range."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from llmplayer_amd import _lib
+from llmplayer_amd import hip_forward_pass as hfp
+from tests import ggml_pack as gp
+from tests.test_block_gpu import NAMES, TYPES
+from tests import test_block_batch_gpu as tbb
+from tests.test_block_batch_gpu import _run_batch
+
+pytestmark = pytest.mark.gpu
+
+
+def _config(hq=8, hkv=2, d=64, **k):
+    return hfp.ModelConfig(hq, hkv, d, 1, architecture=hfp.ARCH_LLAMA, rope_freq_base=500000.0, **k)
+
+
+@pytest.mark.parametrize("t", TYPES, ids=[NAMES[t] for t in TYPES])
+def test_prompt_every_weight_format(t):
+    _run_batch(_config(), 512, 160, 3, 137, (t,) * 4, seed=900 + t, what=f"prompt {NAMES[t]}", batched=True)
+
+
+@pytest.mark.parametrize("K", [136, 255, 256, 257])
+def test_prompt_tile_edges_in_tokens(K):
+    q4, q6 = gp.GGML_Q4_K, gp.GGML_Q6_K
+    _run_batch(_config(), 512, 270, 0, K, (q4, q4, q6, q4), seed=K, what=f"prompt {K} tokens", batched=True)
+
+
+@pytest.mark.parametrize("t", [gp.GGML_Q8_0, gp.GGML_F32, gp.GGML_BF16], ids=["q8_0", "f32", "bf16"])
+def test_prompt_rows_and_columns_off_the_tile(t):
+    # 288 projection rows (4.5 tiles of 64), 352 columns (2.75 chunks of 128)
+    _run_batch(_config(3, 3, 96), 352, 200, 10, 150, (t,) * 4, seed=41 + t, what="prompt 288 x 352", batched=True)
+
+
+@pytest.mark.parametrize("types", [(gp.GGML_Q6_K, gp.GGML_Q6_K, gp.GGML_Q4_K, gp.GGML_Q6_K),
+                                   (gp.GGML_Q3_K, gp.GGML_Q3_K, gp.GGML_Q5_K, gp.GGML_Q5_K),
+                                   (gp.GGML_Q8_0, gp.GGML_Q4_0, gp.GGML_F16, gp.GGML_Q4_K)],
+                         ids=["swapped pair", "q3_k_l", "three launches"])
+def test_prompt_mixes_biases_post_norm_scale(types):
+    _run_batch(_config(), 768, 200, 0, 140, types, seed=sum(types), what="prompt mix", bias=True, post=True,
+               rscale=0.7, batched=True)
+
+
+@pytest.mark.parametrize("K", [31, 33, 64, 130])
+def test_groups_of_16_in_one_launch(K):
+    q4, q6 = gp.GGML_Q4_K, gp.GGML_Q6_K
+    _run_batch(_config(), 512, 160, 7, K, (q4, q4, q6, q4), seed=K, what=f"groups, {K} tokens")
+
+
+@pytest.mark.parametrize("K", [33, 100])
+def test_groups_of_16_in_one_launch_q8_1_input(K):
+    _run_batch(_config(), 512, 160, 7, K, (gp.GGML_Q4_K,) * 4, seed=K, what=f"Q8_1 groups, {K} tokens", q8=True)
+
+
+def test_groups_of_16_in_one_launch_append_what_single_groups_append():
+    """The Q8_1 mode at 150 tokens: K and V rows equal, bit for bit, to those of calls of 16."""
+    c, dim, K = _config(), 512, 150
+    rng = np.random.default_rng(8)
+    x = rng.standard_normal((K, dim)).astype(np.float32)
+    lw, _ = tbb._weights(c, dim, (gp.GGML_Q4_K, gp.GGML_Q4_K, gp.GGML_Q6_K, gp.GGML_Q4_K), rng)
+    rows = []
+    for step in (K, 16):
+        with hfp.HipForwardPass(c, K) as fp:
+            fp.setBlockConfig(dim, input_mode=_lib.LLMP_INPUT_Q8_1)
+            fp.uploadLayerWeights(0, lw)
+            for t in range(0, K, step):
+                fp.uploadXBatch(x[t:t + step])
+                fp.forwardAttentionBlockBatch(0, t, len(x[t:t + step]))
+            rows.append(fp.kv.read(0, 0, K))
+    for a, b in zip(*rows):
+        np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("xs,ws", [(1e6, 1e-6), (1e-20, 1.0), (1.0, 3e4)])
+def test_prompt_far_from_fp16_range(xs, ws):
+    """F32 projections: y = W x to 2^-18 of sum |W||x| per element, whatever their scales (fp32
+    sums of hi/lo products hold ~2^-21)."""
+    c = _config()
+    dim, K = 512, 140
+    rng = np.random.default_rng(3)
+    def mat(r, n, s):
+        return (rng.standard_normal((r, n)) * s / np.sqrt(n)).astype(np.float32)
+    def tensor(w):
+        return hfp.GgufTensor(gp.GGML_F32, w.shape[0], w.shape[1], w.view(np.uint8).reshape(-1))
+    wv = mat(c.kv_dim, dim, ws)
+    zero = np.zeros((c.q_dim, dim), np.float32)
+    x = (rng.standard_normal((K, dim)) * xs).astype(np.float32)
+    with hfp.HipForwardPass(c, K) as fp:
+        fp.setBlockConfig(dim)
+        fp.uploadLayerWeights(0, hfp.TransformerLayerWeights(
+            wq=tensor(zero), wk=tensor(zero[:c.kv_dim]), wv=tensor(wv), wo=tensor(mat(dim, c.q_dim, 1.0))))
+        fp.uploadXBatch(x)
+        fp.forwardAttentionBlockBatch(0, 0, K)
+        _, v = fp.kv.read(0, 0, K)
+    want = x.astype(np.float64) @ wv.T.astype(np.float64)
+    bar = 2.0 ** -18 * (np.abs(x).astype(np.float64) @ np.abs(wv.T).astype(np.float64))
+    assert np.isfinite(v).all() and (np.abs(v - want) <= bar).all()
+
+
+def test_graph_of_a_short_call_outlives_the_growth_of_the_scratch():
+    """A captured 16-token call and a captured 20-token call replay what they computed after a
+    call that needs far more scratch and attention workspace."""
+    c, dim = _config(), 512
+    rng = np.random.default_rng(21)
+    lw, _ = tbb._weights(c, dim, (gp.GGML_Q4_K,) * 4, rng)
+    x = rng.standard_normal((600, dim)).astype(np.float32)
+    with hfp.HipForwardPass(c, 600) as fp:
+        fp.setBlockConfig(dim)
+        fp.uploadLayerWeights(0, lw)
+        bufs = [hfp.DeviceBuffer(n * dim * 4) for n in (16, 20, 600)]
+        try:
+            def put():
+                for b in bufs:
+                    b.upload(x[:b.nbytes // (4 * dim)])
+            graphs, want = [], []
+            for b, n in ((bufs[0], 16), (bufs[1], 20)):
+                put()
+                _lib.call("llmp_attn_block_batch", fp.kv.handle, 0, 0, n, b.ptr, 0)
+                want.append(b.download(np.float32))
+                g = C.c_uint64()
+                _lib.call("llmp_graph_begin", 0)
+                _lib.call("llmp_attn_block_batch", fp.kv.handle, 0, 0, n, b.ptr, 0)
+                _lib.call("llmp_graph_end", 0, C.byref(g))
+                graphs.append(g.value)
+            _lib.call("llmp_attn_block_batch", fp.kv.handle, 0, 0, 600, bufs[2].ptr, 0)
+            for _ in range(3):
+                put()
+                for g, b, w in zip(graphs, bufs, want):
+                    _lib.call("llmp_graph_launch", g, 0)
+                    np.testing.assert_array_equal(b.download(np.float32), w)
+            for g in graphs:
+                _lib.call("llmp_graph_destroy", g)
+        finally:
+            for b in bufs:
+                b.free()
