@@ -16,7 +16,6 @@
 #include <memory>
 #include <mutex>
 #include <string>
-#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -96,7 +95,7 @@ struct KvHandle {
     std::vector<LayerCfg> layers;
     void* prefill_ws = nullptr;   // prefill tile images (grown on demand)
     size_t prefill_ws_bytes = 0;
-    float* prefill_part = nullptr;   // prefill split-K partials (grown on demand)
+    void* prefill_part = nullptr;    // prefill split-K partials (grown on demand)
     size_t prefill_part_bytes = 0;
     float* part_o = nullptr;
     float* part_ml = nullptr;
@@ -108,14 +107,17 @@ struct KvHandle {
     size_t blk_floats = 0;
     void* blkb_buf = nullptr;        // token-batched block scratch (llmp_attn_block_batch)
     size_t blkb_bytes = 0;
-    // The scratch and the attention workspaces of passes of more than kTokBatch tokens, grown on
-    // demand at least twofold.  They are apart from the ones above, and outgrown ones are kept
-    // until the handle goes, so that no graph captured earlier refers to freed memory.
+    // The workspace of the wide multi-token attention, and the scratch and the attention workspaces
+    // of passes of more than kTokBatch tokens, grown on demand at least twofold.  They are apart
+    // from the ones above, and outgrown ones are kept until the handle goes, so that no graph
+    // captured earlier refers to freed memory.
+    void* wide_ws = nullptr;
+    size_t wide_ws_bytes = 0;
     void* many_buf = nullptr;
     size_t many_bytes = 0;
     void* many_ws = nullptr;
     size_t many_ws_bytes = 0;
-    float* many_part = nullptr;
+    void* many_part = nullptr;
     size_t many_part_bytes = 0;
     bool keep_outgrown = false;
     std::vector<void*> outgrown;
@@ -230,6 +232,7 @@ void free_handle(KvHandle* kv) {
     }
     if (kv->blk_buf) (void)hipFree(kv->blk_buf);
     if (kv->blkb_buf) (void)hipFree(kv->blkb_buf);
+    if (kv->wide_ws) (void)hipFree(kv->wide_ws);
     if (kv->many_buf) (void)hipFree(kv->many_buf);
     if (kv->many_ws) (void)hipFree(kv->many_ws);
     if (kv->many_part) (void)hipFree(kv->many_part);
@@ -1426,6 +1429,53 @@ static int enqueue_prefill(KvHandle* kv, int layer, int src_layer, int pos0, int
 
 static int batch_pass(KvHandle* kv, int layer, int pos0, int K, float* xc, uint64_t stream);
 
+// What a multi-token attention call of n tokens needs on one of its two paths: its key tiles (from
+// the first query's window start, or 0, to the last new row), the key splits (0: the wide path does
+// not take the call), and the bytes of the tile images and of the split partials.
+struct PrefillNeed {
+    int TK, tile0, n_tiles, ksplit;
+    size_t ws, part;
+    size_t total() const { return ws + part; }
+};
+static PrefillNeed prefill_need(const KvHandle* kv, const LayerCfg& c, int pos0, int n, bool wide) {
+    const int D = kv->head_dim, Hkv = kv->n_kv_heads, window = layer_window(c);
+    PrefillNeed r{};
+    r.ksplit = wide ? prefill_wide_splits(n, pos0, window, Hkv * c.krep, c.kgroup, D, G().n_cu)
+                    : prefill_key_splits(n, pos0, window, Hkv * c.krep, c.kgroup, D, G().n_cu);
+    if (r.ksplit == 0) return r;
+    r.TK = wide ? prefill_wide_tile_keys(D) : prefill_tile_keys(D);
+    r.tile0 = (window > 0 ? std::max(0, pos0 - window + 1) : 0) / r.TK;
+    r.n_tiles = (pos0 + n - 1) / r.TK - r.tile0 + 1;
+    const size_t tiles = (size_t)Hkv * (size_t)r.n_tiles;
+    if (wide) r.ws = KvHandle::pad256(tiles * prefill_wide_tile_bytes(D));
+    else if (r.ksplit == 1) r.ws = tiles * prefill_tile_bytes(D);   // splits stage straight from the cache
+    if (r.ksplit > 1) r.part = (size_t)r.ksplit * (size_t)n * (size_t)c.n_heads * (size_t)(D + 2) * sizeof(float);
+    return r;
+}
+
+// Grows a workspace to `need` bytes.  The smaller one is freed behind the stream's work on it, or
+// kept (the new one is then at least twice as large, which bounds what is kept).
+static int grow_workspace(KvHandle* kv, void*& buf, size_t& have, size_t need, bool keep, hipStream_t st,
+                          const char* what) {
+    if (need <= have) return LLMP_OK;
+    void* old = buf;
+    if (old && !keep) {
+        LLMP_HIP_CHECK(hipStreamSynchronize(st), "hipStreamSynchronize");
+        (void)hipFree(old);
+        buf = nullptr;
+        have = 0;
+    }
+    if (keep) need = std::max(need, 2 * have);
+    void* mem = nullptr;
+    hipError_t e = hipMalloc(&mem, need);
+    if (e == hipErrorOutOfMemory) return fail(LLMP_ERR_OUT_OF_MEMORY, "llmp_attn_prefill: %zu-byte %s", need, what);
+    LLMP_HIP_CHECK(e, "hipMalloc(prefill workspace)");
+    if (old && keep) kv->outgrown.push_back(old);
+    buf = mem;
+    have = need;
+    return LLMP_OK;
+}
+
 // The attention half of n_tokens tokens at positions pos0 .. pos0+n_tokens-1 over the rows
 // x[t][dim] (LLMEngine.forwardBatch's per-token forwards, LLMEngine.java:1019-1033, with the
 // projections batched as speculative-decoding.md:120-140 plans): per pass of up to kPassTokens
@@ -1477,21 +1527,45 @@ int llmp_attn_block_batch(uint64_t handle, int layer, int pos0, int n_tokens, ui
     int pass = n_tokens < kPassTokens ? n_tokens : kPassTokens;
     if (!kv->blkb_buf || batch_layout(kv, qd, kvd, kTokBatch, true, true).total > kv->blkb_bytes)
         return fail(LLMP_ERR_INVALID_ARG, "llmp_attn_block_batch: layer %d weights not uploaded", layer);
-    const size_t need = pass <= kTokBatch ? 0
-                        : batch_layout(kv, qd, kvd, pass, W[LLMP_W_POST_ATTN_NORM].mem != nullptr,
-                                       kv->blk_input == LLMP_INPUT_Q8_1).total;
-    if (need > kv->many_bytes) {
+    if (pass > kTokBatch) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         LLMP_HIP_CHECK(hipStreamIsCapturing(st, &cap), "hipStreamIsCapturing");
-        const size_t size = std::max(need, 2 * kv->many_bytes);
-        void* mem = nullptr;
-        if (cap == hipStreamCaptureStatusNone && hipMalloc(&mem, size) == hipSuccess) {
-            if (kv->many_buf) kv->outgrown.push_back(kv->many_buf);
-            kv->many_buf = mem;
-            kv->many_bytes = size;
+        const size_t need = batch_layout(kv, qd, kvd, pass, W[LLMP_W_POST_ATTN_NORM].mem != nullptr,
+                                         kv->blk_input == LLMP_INPUT_Q8_1).total;
+        if (cap != hipStreamCaptureStatusNone) {
+            bool fits = need <= kv->many_bytes;
+            for (int t0 = 0; fits && t0 < n_tokens; t0 += pass) {
+                const int n = std::min(pass, n_tokens - t0);
+                const PrefillNeed w = prefill_need(kv, c, pos0 + t0, n, true), p = prefill_need(kv, c, pos0 + t0, n, false);
+                fits = (w.ksplit > 0 && w.total() <= kv->wide_ws_bytes) ||
+                       (p.ws <= kv->many_ws_bytes && p.part <= kv->many_part_bytes) || p.total() <= kv->wide_ws_bytes;
+            }
+            if (!fits) pass = kTokBatch;
         } else {
-            if (cap == hipStreamCaptureStatusNone) (void)hipGetLastError();   // too little memory left
-            pass = kTokBatch;
+            // The attention workspaces of the same call in groups of 16, which a later captured
+            // call may take.
+            size_t ws = 0, part = 0;
+            for (int t0 = 0; t0 < n_tokens; t0 += kTokBatch) {
+                const PrefillNeed p = prefill_need(kv, c, pos0 + t0, std::min(kTokBatch, n_tokens - t0), false);
+                ws = std::max(ws, p.ws);
+                part = std::max(part, p.part);
+            }
+            if (int rc = grow_workspace(kv, kv->prefill_ws, kv->prefill_ws_bytes, ws, true, st, "tile workspace"))
+                return rc;
+            if (int rc = grow_workspace(kv, kv->prefill_part, kv->prefill_part_bytes, part, true, st, "split workspace"))
+                return rc;
+            if (need > kv->many_bytes) {
+                const size_t size = std::max(need, 2 * kv->many_bytes);
+                void* mem = nullptr;
+                if (hipMalloc(&mem, size) == hipSuccess) {
+                    if (kv->many_buf) kv->outgrown.push_back(kv->many_buf);
+                    kv->many_buf = mem;
+                    kv->many_bytes = size;
+                } else {
+                    (void)hipGetLastError();   // too little memory left
+                    pass = kTokBatch;
+                }
+            }
         }
     }
     for (int t0 = 0; t0 < n_tokens; t0 += pass)
@@ -1886,7 +1960,7 @@ static int enqueue_prefill(KvHandle* kv, int layer, int src_layer, int pos0, int
     a.Hq = c.n_heads;
     a.Hkv = Hkv;
     a.rope_type = c.rope_type;
-    a.window = (c.window > 0 && !c.is_global) ? c.window : 0;
+    a.window = layer_window(c);
     a.eps = c.eps;
     const float scale = c.scale > 0.0f ? c.scale : (float)(1.0 / std::sqrt((double)D));
     const float log2e = 1.4426950408889634f;
@@ -1899,70 +1973,53 @@ static int enqueue_prefill(KvHandle* kv, int layer, int src_layer, int pos0, int
         a.qk_scale = scale * log2e;
     }
     hipStream_t st = pick_stream(stream);
-    // Key tiles any query of this call attends: from the first query's window start (or 0) to
-    // the last prompt row.  Their images live in the handle's workspace, grown when a call
-    // needs more (a growth synchronises the device; the size only depends on the row range).
-    const int kbeg_min = a.window > 0 ? std::max(0, pos0 - a.window + 1) : 0;
-    int TK = prefill_tile_keys(D);
-    int tile0 = kbeg_min / TK;
-    int n_tiles = (pos0 + n_tokens - 1) / TK - tile0 + 1;
-    int ksplit = prefill_key_splits(n_tokens, pos0, a.window, Hkv * c.krep, group, D, G().n_cu);
-    const size_t part_1 = (size_t)n_tokens * (size_t)c.n_heads * (size_t)(D + 2) * sizeof(float);
-    size_t ws_bytes = ksplit == 1 ? (size_t)Hkv * (size_t)n_tiles * prefill_tile_bytes(D) : 0;
-    size_t part_bytes = ksplit > 1 ? (size_t)ksplit * part_1 : 0;
-    // The static array's limit counts this plan's workspace, on either path.
-    if (use_static && ws_bytes + part_bytes > (size_t)LLMP_PREFILL_STATIC_BYTES)
-        return fail(LLMP_ERR_INVALID_ARG,
-                    "llmp_attn_prefill_f32_static: the call needs %zu bytes of workspace; the "
-                    "static scratch holds %u (fewer tokens per call, or llmp_attn_prefill_f32)",
-                    ws_bytes + part_bytes, (unsigned)LLMP_PREFILL_STATIC_BYTES);
-    const int wide = prefill_wide_splits(n_tokens, pos0, a.window, Hkv * c.krep, group, D, G().n_cu);
+    const PrefillNeed narrow = prefill_need(kv, c, pos0, n_tokens, false);
+    const PrefillNeed wide = prefill_need(kv, c, pos0, n_tokens, true);
     bool use_wide = false;
-    if (wide > 0) {
-        const int wtk = prefill_wide_tile_keys(D), wt0 = kbeg_min / wtk;
-        const int wnt = (pos0 + n_tokens - 1) / wtk - wt0 + 1;
-        const size_t wws = KvHandle::pad256((size_t)Hkv * (size_t)wnt * prefill_wide_tile_bytes(D));
-        const size_t wpart = wide > 1 ? (size_t)wide * part_1 : 0;
-        if (!use_static || wws + wpart <= (size_t)LLMP_PREFILL_STATIC_BYTES) {
-            use_wide = true;
-            TK = wtk, tile0 = wt0, n_tiles = wnt, ksplit = wide, ws_bytes = wws, part_bytes = wpart;
-        }
-    }
-    void* ws = kv->prefill_ws;
+    void* ws = nullptr;
     if (use_static) {
-        // The whole workspace (tile images, split-K partials) in the static array: no
-        // allocation, no profiling events.
+        // The whole workspace in the static array: no allocation, no profiling events.  Its limit
+        // counts the narrow path's workspace, on either path.
+        if (narrow.total() > (size_t)LLMP_PREFILL_STATIC_BYTES)
+            return fail(LLMP_ERR_INVALID_ARG,
+                        "llmp_attn_prefill_f32_static: the call needs %zu bytes of workspace; the "
+                        "static scratch holds %u (fewer tokens per call, or llmp_attn_prefill_f32)",
+                        narrow.total(), (unsigned)LLMP_PREFILL_STATIC_BYTES);
         ws = G().scratch;
         if (!ws) return fail(LLMP_ERR_NOT_INIT, "llmp_attn_prefill_f32_static: no scratch address");
-        a.part_o = reinterpret_cast<float*>(static_cast<char*>(ws) + ws_bytes);
+        use_wide = wide.ksplit > 0 && wide.total() <= (size_t)LLMP_PREFILL_STATIC_BYTES;
+        a.part_o = reinterpret_cast<float*>(static_cast<char*>(ws) + (use_wide ? wide.ws : narrow.ws));
     } else {
-        // A growth frees the smaller workspace behind the stream's work on it, or keeps it
-        // (KvHandle::keep_outgrown).
-        auto grow = [&](auto*& buf, size_t& have, size_t need, const char* what) -> int {
-            if (need <= have) return LLMP_OK;
-            void* old = buf;
-            if (old && !kv->keep_outgrown) {
-                LLMP_HIP_CHECK(hipStreamSynchronize(st), "hipStreamSynchronize");
-                (void)hipFree(old);
-                buf = nullptr;
-                have = 0;
-            }
-            if (kv->keep_outgrown) need = std::max(need, 2 * have);
-            void* mem = nullptr;
-            hipError_t e = hipMalloc(&mem, need);
-            if (e == hipErrorOutOfMemory) return fail(LLMP_ERR_OUT_OF_MEMORY, "llmp_attn_prefill: %zu-byte %s", need, what);
-            LLMP_HIP_CHECK(e, "hipMalloc(prefill workspace)");
-            if (old && kv->keep_outgrown) kv->outgrown.push_back(old);
-            buf = static_cast<std::remove_reference_t<decltype(buf)>>(mem);
-            have = need;
-            return LLMP_OK;
-        };
-        if (int rc = grow(kv->prefill_ws, kv->prefill_ws_bytes, ws_bytes, "tile workspace")) return rc;
-        ws = kv->prefill_ws;
-        // Key splits (chunks whose query blocks leave CUs idle) and their partials buffer.
-        if (int rc = grow(kv->prefill_part, kv->prefill_part_bytes, part_bytes, "split workspace")) return rc;
-        a.part_o = kv->prefill_part;
+        // Each path has its own workspace.  The wide one is grown to what the call would need on
+        // either path, so that whatever a call prepares a later captured one for does not depend
+        // on its path: a captured narrow call whose own workspace is too small takes it.  A
+        // captured call whose wide workspace would have to grow, or one that finds no memory for
+        // it, takes the narrow path.
+        const size_t wide_need = wide.ksplit > 0 ? std::max(wide.total(), narrow.total()) : 0;
+        const bool own = narrow.ws <= kv->prefill_ws_bytes && narrow.part <= kv->prefill_part_bytes;
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (wide_need > kv->wide_ws_bytes || !own) LLMP_HIP_CHECK(hipStreamIsCapturing(st, &cap), "hipStreamIsCapturing");
+        const bool eager = cap == hipStreamCaptureStatusNone;
+        if (wide_need > kv->wide_ws_bytes && eager &&
+            grow_workspace(kv, kv->wide_ws, kv->wide_ws_bytes, wide_need, true, st, "wide workspace") != LLMP_OK)
+            (void)hipGetLastError();
+        use_wide = wide.ksplit > 0 && wide.total() <= kv->wide_ws_bytes;
+        if (use_wide || (!own && !eager && narrow.total() <= kv->wide_ws_bytes)) {
+            ws = kv->wide_ws;
+            a.part_o = reinterpret_cast<float*>(static_cast<char*>(ws) + (use_wide ? wide.ws : narrow.ws));
+        } else {
+            if (int rc = grow_workspace(kv, kv->prefill_ws, kv->prefill_ws_bytes, narrow.ws, kv->keep_outgrown, st,
+                                        "tile workspace"))
+                return rc;
+            if (int rc = grow_workspace(kv, kv->prefill_part, kv->prefill_part_bytes, narrow.part, kv->keep_outgrown,
+                                        st, "split workspace"))
+                return rc;
+            ws = kv->prefill_ws;
+            a.part_o = static_cast<float*>(kv->prefill_part);
+        }
     }
+    const PrefillNeed& plan = use_wide ? wide : narrow;
+    const int tile0 = plan.tile0, n_tiles = plan.n_tiles, ksplit = plan.ksplit;
     if (ksplit > 1) a.part_ml = a.part_o + (size_t)ksplit * n_tokens * c.n_heads * D;
     const bool prof = kv->prof_on && !use_static;
     hipEvent_t e0 = nullptr, e1 = nullptr, e2 = nullptr, e3 = nullptr;

@@ -1,5 +1,5 @@
 // Multi-token attention on 32x32 matrix tiles: the path of calls whose key tiles are each read
-// by several workgroups (prefill_wide_plan); shorter chunks stay on prefill_kernels.h.
+// by several workgroups (prefill_wide_splits); shorter chunks stay on prefill_kernels.h.
 //
 // One KV head's queries are flattened to columns c = token * G + head (G query heads per KV
 // head), so a workgroup of 4 waves takes 128 consecutive columns whatever G is and no MFMA

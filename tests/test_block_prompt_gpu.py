@@ -140,3 +140,44 @@ def test_graph_of_a_short_call_outlives_the_growth_of_the_scratch():
         finally:
             for b in bufs:
                 b.free()
+
+
+@pytest.mark.parametrize("first", [(0, 300), (900, 40)])
+def test_capture_beyond_the_prepared_workspaces_runs_in_groups(first):
+    """A captured call of more tokens, or at a later position, than the eager calls before it had:
+    in groups of 16 if a workspace would have to grow, with the eager call's result to rounding."""
+    c, dim, pos0, K = _config(), 512, 600, 300
+    rng = np.random.default_rng(22)
+    lw, _ = tbb._weights(c, dim, (gp.GGML_Q4_K,) * 4, rng)
+    x = rng.standard_normal((K, dim)).astype(np.float32)
+    with hfp.HipForwardPass(c, 1000) as fp:
+        fp.setBlockConfig(dim)
+        fp.uploadLayerWeights(0, lw)
+        rows = rng.standard_normal((2, 1000, c.kv_dim)).astype(np.float32)
+        fp.kv.write(0, 0, rows[0], rows[1])
+        buf = hfp.DeviceBuffer(x.nbytes)
+        try:
+            def call(pos, n):
+                _lib.call("llmp_attn_block_batch", fp.kv.handle, 0, pos, n, buf.ptr, 0)
+            buf.upload(x)
+            call(*first)
+            call(pos0 + K - 16, 16)   # the groups' own workspaces
+            fp.kv.write(0, 0, rows[0], rows[1])
+            g = C.c_uint64()
+            _lib.call("llmp_graph_begin", 0)
+            call(pos0, K)
+            _lib.call("llmp_graph_end", 0, C.byref(g))
+            got = []
+            for _ in range(3):
+                buf.upload(x)
+                _lib.call("llmp_graph_launch", g.value, 0)
+                _lib.call("llmp_stream_sync", 0)
+                got.append(buf.download(np.float32, x.size))
+                buf.upload(x)
+                call(pos0, K)
+            want = buf.download(np.float32, x.size)
+            _lib.call("llmp_graph_destroy", g.value)
+        finally:
+            buf.free()
+    for y in got:   # fp32 sums in another order: the bar of the batched blocks
+        assert np.abs(y - want).max() <= 1e-4

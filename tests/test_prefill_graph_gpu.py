@@ -107,3 +107,40 @@ def test_verification_graph_replays(q8):
         finally:
             for b in bufs:
                 b.free()
+
+
+def test_capture_of_a_shorter_call_after_a_longer_one():
+    """A call of 60 tokens captured without one of its own before: a longer call (on the wide path)
+    has prepared the workspaces of both paths."""
+    import ctypes as C
+    c = hfp.ModelConfig(24, 8, 128, 1, architecture=hfp.ARCH_LLAMA, rope_freq_base=500000.0)
+    pos0, P, K = 2000, 300, 60
+    rng = np.random.default_rng(63)
+    with hfp.HipForwardPass(c, pos0 + P) as fp:
+        fp.kv.write(0, 0, rng.standard_normal((pos0, c.kv_dim), dtype=np.float32) * F32(0.5),
+                    rng.standard_normal((pos0, c.kv_dim), dtype=np.float32))
+        bufs = [hfp.DeviceBuffer(P * n * 4) for n in (c.q_dim, c.kv_dim, c.kv_dim, c.q_dim)]
+        try:
+            for b in bufs[:3]:
+                b.upload(rng.standard_normal(b.nbytes // 4, dtype=np.float32))
+
+            def call(n):
+                _lib.call("llmp_attn_prefill_f32", fp.kv.handle, 0, pos0, n, bufs[0].ptr, bufs[1].ptr,
+                          bufs[2].ptr, 0, bufs[3].ptr, 0)
+            call(P)
+            g = C.c_uint64()
+            _lib.call("llmp_graph_begin", 0)
+            call(K)
+            _lib.call("llmp_graph_end", 0, C.byref(g))
+            call(K)
+            want = bufs[3].download(np.float32, K * c.q_dim)
+            for _ in range(3):
+                bufs[3].upload(np.zeros(P * c.q_dim, np.float32))
+                _lib.call("llmp_graph_launch", g.value, 0)
+                _lib.call("llmp_stream_sync", 0)
+                np.testing.assert_array_equal(bufs[3].download(np.float32, K * c.q_dim), want)
+                call(P)
+            _lib.call("llmp_graph_destroy", g.value)
+        finally:
+            for b in bufs:
+                b.free()
