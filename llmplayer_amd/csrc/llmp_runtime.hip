@@ -48,8 +48,7 @@ struct DevWeight {
     int rows = 0, cols = 0;
     void* mem = nullptr;
     gk::WPlanes planes{};
-    int* rexp = nullptr;   // matrices: [rows] exponents of the many-token projections (in mem),
-    bool rexp_set = false; // filled by the first of them
+    int* rexp = nullptr;   // matrices: [rows] exponents of the many-token projections (in mem)
     // The token-batched projections split fp32 and bf16 weights into fp16 parts: false when
     // some weight reaches fp16's largest magnitude, 65504, or for a type proj_tok_supported
     // rejects (llmp_attn_block_batch then runs the tokens one by one, on the fp32 single-token
@@ -1268,7 +1267,14 @@ int llmp_layer_weight(uint64_t handle, int layer, int slot, int ggml_type, int r
         w.planes.p[i] = static_cast<const unsigned char*>(w.mem) + off[i];
         w.planes.pitch[i] = (long long)pitch[i];
     }
-    if (!vec) w.rexp = reinterpret_cast<int*>(static_cast<char*>(w.mem) + rexp_off);
+    if (!vec && proj_tok_supported(ggml_type)) {
+        // The row exponents, behind the upload and complete when this returns (any stream may read
+        // them).  A first call of many tokens that computed them stalled its stream, and a captured
+        // one could not: it kept the 16-token projections for the life of the graph.
+        w.rexp = reinterpret_cast<int*>(static_cast<char*>(w.mem) + rexp_off);
+        LLMP_HIP_CHECK(launch_weight_range(w.planes, ggml_type, rows, cols, w.rexp, nullptr), "weight range launch");
+        LLMP_HIP_CHECK(hipStreamSynchronize(nullptr), "hipStreamSynchronize");
+    }
     // Block scratch: q | k | v, the attention output and the Wo output (kept per handle).
     const size_t need = (size_t)(qd + 2 * kvd) + (size_t)qd + (size_t)dim + 64;
     if (need > kv->blk_floats) {
@@ -1575,32 +1581,6 @@ int llmp_attn_block_batch(uint64_t handle, int layer, int pos0, int n_tokens, ui
     return LLMP_OK;
 }
 
-// The row exponents of a layer's matrices, computed by its first call of many tokens and complete
-// when this returns, so that any stream may read them.  Under capture nothing can be waited for:
-// *gemm becomes false where some are missing (the groups of 16 need none).
-static int row_exponents(DevWeight* W, bool merged, hipStream_t st, bool* gemm) {
-    bool launched = false;
-    for (int slot = LLMP_W_Q; slot <= LLMP_W_O; ++slot) {
-        DevWeight& w = W[slot];
-        const bool used = slot == LLMP_W_O || (slot == LLMP_W_QKV) == merged;
-        if (!used || w.rexp_set) continue;
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        LLMP_HIP_CHECK(hipStreamIsCapturing(st, &cap), "hipStreamIsCapturing");
-        if (cap != hipStreamCaptureStatusNone) {
-            *gemm = false;
-            return LLMP_OK;
-        }
-        LLMP_HIP_CHECK(launch_weight_range(w.planes, w.type, w.rows, w.cols, w.rexp, st), "weight range launch");
-        launched = true;
-    }
-    if (launched) {
-        LLMP_HIP_CHECK(hipStreamSynchronize(st), "hipStreamSynchronize");
-        for (int slot = LLMP_W_Q; slot <= LLMP_W_O; ++slot)
-            if (slot == LLMP_W_O || (slot == LLMP_W_QKV) == merged) W[slot].rexp_set = true;
-    }
-    return LLMP_OK;
-}
-
 // One pass of llmp_attn_block_batch over K tokens (rows xc), within the handle's scratch.
 static int batch_pass(KvHandle* kv, int layer, int pos0, int K, float* xc, uint64_t stream) {
     // A group of one token takes the single-token launches, which are faster for it (27 against 49
@@ -1616,9 +1596,7 @@ static int batch_pass(KvHandle* kv, int layer, int pos0, int K, float* xc, uint6
     const int D = kv->head_dim, qd = c.n_heads * D, kvd = kv->n_kv_heads * D, dim = kv->blk_dim;
     const bool q8 = kv->blk_input == LLMP_INPUT_Q8_1;
     hipStream_t st = pick_stream(stream);
-    bool gemm = !q8 && K >= kGemmTokens;
-    if (gemm)
-        if (int rc = row_exponents(kv->layers[(size_t)layer].w, merged, st, &gemm)) return rc;
+    const bool gemm = !q8 && K >= kGemmTokens;
     const BatchLayout L = batch_layout(kv, qd, kvd, K, W[LLMP_W_POST_ATTN_NORM].mem != nullptr, q8);
     const bool many = K > kTokBatch;
     char* base = static_cast<char*>(many ? kv->many_buf : kv->blkb_buf);

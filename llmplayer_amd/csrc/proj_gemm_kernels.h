@@ -15,7 +15,7 @@
 // 178 us for the whole call at 96 tokens, where a stage's latency is all there is.
 //
 // Precision.  A weight is w * 2^E_row = hi + lo with E_row from the row's largest magnitude
-// (weight_range_kernel, once per weight), so hi + lo holds it to 2^-22 down to 2^-17 of the row's
+// (weight_range_kernel, at upload), so hi + lo holds it to 2^-22 down to 2^-17 of the row's
 // largest; an input likewise with its token's exponent.  Products are hi*hi + hi*lo + lo*hi; each
 // 128-column chunk is summed by the matrix unit from zero and added to the running sum in fp32,
 // which keeps that chain as short as the 16-token kernel's.  F16 and BF16 rows have no lo part.
@@ -123,7 +123,7 @@ __device__ __forceinline__ void chunk_table(const typename F::Raw& raw, float* t
     }
 }
 
-// E_row of rows 16 blockIdx.x .. +15 of a matrix (once per weight, by its first use).
+// E_row of rows 16 blockIdx.x .. +15 of a matrix (once per weight, at its upload).
 template <class F>
 __global__ __launch_bounds__(kThreads) void weight_range_kernel(WPlanes w, int cols, int* rexp) {
     __shared__ float s_tab[kWaves][16 * (F::TAB > 0 ? F::TAB : 1)];

@@ -181,3 +181,36 @@ def test_capture_beyond_the_prepared_workspaces_runs_in_groups(first):
             buf.free()
     for y in got:   # fp32 sums in another order: the bar of the batched blocks
         assert np.abs(y - want).max() <= 1e-4
+
+
+def test_a_layer_captured_before_it_ever_ran_takes_the_tiled_projections():
+    """Two layers of the same weights: the captured call of the one that never ran replays, bit for
+    bit, what the other's eager call computed."""
+    c = hfp.ModelConfig(8, 2, 64, 2, architecture=hfp.ARCH_LLAMA, rope_freq_base=500000.0)
+    dim, K = 512, 300
+    rng = np.random.default_rng(4)
+    lw, _ = tbb._weights(c, dim, (gp.GGML_Q4_K,) * 4, rng)
+    x = rng.standard_normal((K, dim)).astype(np.float32)
+    with hfp.HipForwardPass(c, K) as fp:
+        fp.setBlockConfig(dim)
+        for layer in (0, 1):
+            fp.uploadLayerWeights(layer, lw)
+        buf = hfp.DeviceBuffer(x.nbytes)
+        try:
+            def call(layer):
+                _lib.call("llmp_attn_block_batch", fp.kv.handle, layer, 0, K, buf.ptr, 0)
+            buf.upload(x)
+            call(0)   # the handle's scratch and workspaces
+            want = buf.download(np.float32)
+            g = C.c_uint64()
+            _lib.call("llmp_graph_begin", 0)
+            call(1)
+            _lib.call("llmp_graph_end", 0, C.byref(g))
+            for _ in range(3):
+                buf.upload(x)
+                _lib.call("llmp_graph_launch", g.value, 0)
+                np.testing.assert_array_equal(buf.download(np.float32), want)
+                call(0)
+            _lib.call("llmp_graph_destroy", g.value)
+        finally:
+            buf.free()
