@@ -253,9 +253,9 @@ int llmp_decode_plan(uint64_t handle, int layer, int position, int splits, int *
  * "thread local").  Profiling must be off while capturing.  A graph holds the device addresses
  * its launches had at capture time.  Decode's split workspace is allocated once by
  * llmp_kv_create and never moves, but set-up calls (llmp_layer_config, llmp_layer_sinks,
- * llmp_rope_upload, llmp_layer_weight) and a prefill call that grows the handle's prefill
- * workspace can free memory an earlier graph refers to: capture after set-up, and capture
- * again after any of them. */
+ * llmp_rope_upload, llmp_layer_weight) can free memory an earlier graph refers to: capture after
+ * set-up, and capture again after any of them.  (Prefill workspaces that a captured call uses are
+ * kept until the handle is destroyed, also where later calls outgrow them.) */
 int llmp_graph_begin(uint64_t stream);
 /* Stop capturing and instantiate the graph; *graph receives an executable-graph handle. */
 int llmp_graph_end(uint64_t stream, uint64_t *graph);
@@ -279,8 +279,8 @@ int llmp_graph_destroy(uint64_t graph);
  * Partial RoPE (rotated dims < head_dim, NORMAL or NEOX pairs) is applied as in decode.
  * The handle keeps a workspace for the key tiles a call attends (fp16 hi/lo images of K and
  * V: about 9 bytes per key, KV head and head_dim element); a call that needs more than any
- * earlier call grows it (hipFree + hipMalloc: such a call cannot be captured in a graph, and
- * graphs captured before it must not be replayed after it). */
+ * earlier call grows it, at least twofold (such a call cannot be captured in a graph).  The
+ * smaller one is freed, or kept for a graph that a call on it was captured into. */
 int llmp_attn_prefill(uint64_t handle, int layer, int pos0, int n_tokens, uint64_t q,
                       uint64_t k, uint64_t v, uint64_t out, uint64_t stream);
 /* llmp_attn_prefill with an optional output gate (device fp32 [n_tokens][n_heads*head_dim],
@@ -411,11 +411,10 @@ int llmp_attn_block(uint64_t handle, int layer, int position, uint64_t d_positio
  * LLMP_INPUT_Q8_1 mode the routed types take each token's Q8_1 input as llmp_attn_block forms it
  * (the same staged norm and quantiser) and exact integer block dots on the matrix cores, and Wo
  * the quantised attention output.  At head_dim 80 (no prefill kernel) and for layers whose fp32
- * or bf16 weights reach 65504, the tokens run one llmp_attn_block call each.  A call of up to 16
- * tokens may grow the handle's prefill workspace, as llmp_attn_prefill_f32 does (not for use
- * under graph capture then); longer ones have a scratch and workspaces of their own, which grow
- * too: outgrown ones are kept until the handle is destroyed, so graphs captured before stay
- * valid, and a captured call whose scratch would have to grow runs in groups of 16 tokens. */
+ * or bf16 weights reach 65504, the tokens run one llmp_attn_block call each.  The call may grow the
+ * handle's prefill workspaces, as llmp_attn_prefill_f32 does, and from 17 tokens on a scratch of
+ * its own; what captured calls use is kept until the handle is destroyed, so graphs captured
+ * before stay valid.  A captured call whose scratch would have to grow runs in groups of 16 tokens. */
 int llmp_attn_block_batch(uint64_t handle, int layer, int pos0, int n_tokens, uint64_t x,
                           uint64_t stream);
 

@@ -6,6 +6,7 @@
 #include "prefill_kernels.h"
 #include "gemv_kernels.h"
 #include "proj_gemm_kernels.h"
+#include "workspace.h"
 
 #include <algorithm>
 #include <cmath>
@@ -92,10 +93,11 @@ struct KvHandle {
     size_t plane_floats = 0;  // floats of one K or V plane of one layer
     RopeTable rope[2];
     std::vector<LayerCfg> layers;
-    void* prefill_ws = nullptr;   // prefill tile images (grown on demand)
-    size_t prefill_ws_bytes = 0;
-    void* prefill_part = nullptr;    // prefill split-K partials (grown on demand)
-    size_t prefill_part_bytes = 0;
+    Workspace prefill_ws;            // prefill tile images
+    Workspace prefill_part;          // prefill split-K partials
+    Workspace wide_ws;               // tile images and partials of the wide multi-token attention
+    Workspace many_buf;              // scratch of llmp_attn_block_batch passes of more than kTokBatch tokens
+    std::vector<void*> outgrown;     // kept for captured graphs (workspace.h)
     float* part_o = nullptr;
     float* part_ml = nullptr;
     int* done = nullptr;             // per virtual KV head: the decode split counters (zero between calls)
@@ -106,20 +108,6 @@ struct KvHandle {
     size_t blk_floats = 0;
     void* blkb_buf = nullptr;        // token-batched block scratch (llmp_attn_block_batch)
     size_t blkb_bytes = 0;
-    // The workspace of the wide multi-token attention, and the scratch and the attention workspaces
-    // of passes of more than kTokBatch tokens, grown on demand at least twofold.  They are apart
-    // from the ones above, and outgrown ones are kept until the handle goes, so that no graph
-    // captured earlier refers to freed memory.
-    void* wide_ws = nullptr;
-    size_t wide_ws_bytes = 0;
-    void* many_buf = nullptr;
-    size_t many_bytes = 0;
-    void* many_ws = nullptr;
-    size_t many_ws_bytes = 0;
-    void* many_part = nullptr;
-    size_t many_part_bytes = 0;
-    bool keep_outgrown = false;
-    std::vector<void*> outgrown;
     size_t part_slots = 0;    // (split, query head) slots the workspace holds
     bool prof_on = false;
     std::vector<ProfPair> prof_pending[LLMP_PROF_KINDS];
@@ -231,16 +219,12 @@ void free_handle(KvHandle* kv) {
     }
     if (kv->blk_buf) (void)hipFree(kv->blk_buf);
     if (kv->blkb_buf) (void)hipFree(kv->blkb_buf);
-    if (kv->wide_ws) (void)hipFree(kv->wide_ws);
-    if (kv->many_buf) (void)hipFree(kv->many_buf);
-    if (kv->many_ws) (void)hipFree(kv->many_ws);
-    if (kv->many_part) (void)hipFree(kv->many_part);
+    for (Workspace* w : {&kv->prefill_ws, &kv->prefill_part, &kv->wide_ws, &kv->many_buf})
+        if (w->mem) (void)hipFree(w->mem);
     for (void* p : kv->outgrown) (void)hipFree(p);
     if (kv->part_o) (void)hipFree(kv->part_o);
     if (kv->part_ml) (void)hipFree(kv->part_ml);
     if (kv->done) (void)hipFree(kv->done);
-    if (kv->prefill_ws) (void)hipFree(kv->prefill_ws);
-    if (kv->prefill_part) (void)hipFree(kv->prefill_part);
     for (auto& v : kv->prof_pending)
         for (auto& p : v) {
             (void)hipEventDestroy(p.begin);
@@ -1459,27 +1443,41 @@ static PrefillNeed prefill_need(const KvHandle* kv, const LayerCfg& c, int pos0,
     return r;
 }
 
-// Grows a workspace to `need` bytes.  The smaller one is freed behind the stream's work on it, or
-// kept (the new one is then at least twice as large, which bounds what is kept).
-static int grow_workspace(KvHandle* kv, void*& buf, size_t& have, size_t need, bool keep, hipStream_t st,
-                          const char* what) {
-    if (need <= have) return LLMP_OK;
-    void* old = buf;
-    if (old && !keep) {
-        LLMP_HIP_CHECK(hipStreamSynchronize(st), "hipStreamSynchronize");
-        (void)hipFree(old);
-        buf = nullptr;
-        have = 0;
-    }
-    if (keep) need = std::max(need, 2 * have);
-    void* mem = nullptr;
-    hipError_t e = hipMalloc(&mem, need);
-    if (e == hipErrorOutOfMemory) return fail(LLMP_ERR_OUT_OF_MEMORY, "llmp_attn_prefill: %zu-byte %s", need, what);
-    LLMP_HIP_CHECK(e, "hipMalloc(prefill workspace)");
-    if (old && keep) kv->outgrown.push_back(old);
-    buf = mem;
-    have = need;
+// Whether work enqueued on the stream now is recorded into a graph.
+static int stream_capturing(hipStream_t st, bool* capturing) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    LLMP_HIP_CHECK(hipStreamIsCapturing(st, &cap), "hipStreamIsCapturing");
+    *capturing = cap != hipStreamCaptureStatusNone;
     return LLMP_OK;
+}
+
+// Workspace::grow on the device; `st` is the stream that works on the present buffer.
+struct DeviceMemory {
+    hipStream_t st;
+    hipError_t err = hipSuccess;
+    Alloc alloc(size_t bytes, void** mem) {
+        err = hipMalloc(mem, bytes);
+        if (err == hipSuccess) return Alloc::ok;
+        (void)hipGetLastError();
+        return err == hipErrorOutOfMemory ? Alloc::no_memory : Alloc::failed;
+    }
+    void release(void* mem) {
+        (void)hipStreamSynchronize(st);
+        (void)hipFree(mem);
+    }
+};
+static int grow_workspace(KvHandle* kv, Workspace& w, size_t need, bool capturing, hipStream_t st, const char* what) {
+    DeviceMemory dev{st};
+    switch (w.grow(need, capturing, kv->outgrown, dev)) {
+    case Alloc::ok: return LLMP_OK;
+    case Alloc::no_memory: return fail(LLMP_ERR_OUT_OF_MEMORY, "llmp_attn_prefill: %zu-byte %s", need, what);
+    default: LLMP_HIP_CHECK(dev.err, "hipMalloc(prefill workspace)"); return LLMP_OK;
+    }
+}
+// The same for a workspace that the call can do without: false where there is no memory for it.
+static bool try_grow_workspace(KvHandle* kv, Workspace& w, size_t need, hipStream_t st) {
+    DeviceMemory dev{st};
+    return w.try_grow(need, kv->outgrown, dev);
 }
 
 // The attention half of n_tokens tokens at positions pos0 .. pos0+n_tokens-1 over the rows
@@ -1534,44 +1532,32 @@ int llmp_attn_block_batch(uint64_t handle, int layer, int pos0, int n_tokens, ui
     if (!kv->blkb_buf || batch_layout(kv, qd, kvd, kTokBatch, true, true).total > kv->blkb_bytes)
         return fail(LLMP_ERR_INVALID_ARG, "llmp_attn_block_batch: layer %d weights not uploaded", layer);
     if (pass > kTokBatch) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        LLMP_HIP_CHECK(hipStreamIsCapturing(st, &cap), "hipStreamIsCapturing");
+        bool capturing;
+        if (int rc = stream_capturing(st, &capturing)) return rc;
         const size_t need = batch_layout(kv, qd, kvd, pass, W[LLMP_W_POST_ATTN_NORM].mem != nullptr,
                                          kv->blk_input == LLMP_INPUT_Q8_1).total;
-        if (cap != hipStreamCaptureStatusNone) {
-            bool fits = need <= kv->many_bytes;
+        if (capturing) {
+            bool fits = need <= kv->many_buf.bytes;
             for (int t0 = 0; fits && t0 < n_tokens; t0 += pass) {
                 const int n = std::min(pass, n_tokens - t0);
                 const PrefillNeed w = prefill_need(kv, c, pos0 + t0, n, true), p = prefill_need(kv, c, pos0 + t0, n, false);
-                fits = (w.ksplit > 0 && w.total() <= kv->wide_ws_bytes) ||
-                       (p.ws <= kv->many_ws_bytes && p.part <= kv->many_part_bytes) || p.total() <= kv->wide_ws_bytes;
+                fits = (w.ksplit > 0 && w.total() <= kv->wide_ws.bytes) ||
+                       (p.ws <= kv->prefill_ws.bytes && p.part <= kv->prefill_part.bytes) || p.total() <= kv->wide_ws.bytes;
             }
-            if (!fits) pass = kTokBatch;
+            if (fits) kv->many_buf.captured = true;
+            else pass = kTokBatch;
         } else {
             // The attention workspaces of the same call in groups of 16, which a later captured
-            // call may take.
+            // call may take (this one does without them).
             size_t ws = 0, part = 0;
             for (int t0 = 0; t0 < n_tokens; t0 += kTokBatch) {
                 const PrefillNeed p = prefill_need(kv, c, pos0 + t0, std::min(kTokBatch, n_tokens - t0), false);
                 ws = std::max(ws, p.ws);
                 part = std::max(part, p.part);
             }
-            if (int rc = grow_workspace(kv, kv->prefill_ws, kv->prefill_ws_bytes, ws, true, st, "tile workspace"))
-                return rc;
-            if (int rc = grow_workspace(kv, kv->prefill_part, kv->prefill_part_bytes, part, true, st, "split workspace"))
-                return rc;
-            if (need > kv->many_bytes) {
-                const size_t size = std::max(need, 2 * kv->many_bytes);
-                void* mem = nullptr;
-                if (hipMalloc(&mem, size) == hipSuccess) {
-                    if (kv->many_buf) kv->outgrown.push_back(kv->many_buf);
-                    kv->many_buf = mem;
-                    kv->many_bytes = size;
-                } else {
-                    (void)hipGetLastError();   // too little memory left
-                    pass = kTokBatch;
-                }
-            }
+            (void)try_grow_workspace(kv, kv->prefill_ws, ws, st);
+            (void)try_grow_workspace(kv, kv->prefill_part, part, st);
+            if (!try_grow_workspace(kv, kv->many_buf, need, st)) pass = kTokBatch;
         }
     }
     for (int t0 = 0; t0 < n_tokens; t0 += pass)
@@ -1598,8 +1584,7 @@ static int batch_pass(KvHandle* kv, int layer, int pos0, int K, float* xc, uint6
     hipStream_t st = pick_stream(stream);
     const bool gemm = !q8 && K >= kGemmTokens;
     const BatchLayout L = batch_layout(kv, qd, kvd, K, W[LLMP_W_POST_ATTN_NORM].mem != nullptr, q8);
-    const bool many = K > kTokBatch;
-    char* base = static_cast<char*>(many ? kv->many_buf : kv->blkb_buf);
+    char* base = static_cast<char*>(K > kTokBatch ? kv->many_buf.mem : kv->blkb_buf);
     float* qb = reinterpret_cast<float*>(base + L.q);
     float* kb = reinterpret_cast<float*>(base + L.k);
     float* vb = reinterpret_cast<float*>(base + L.v);
@@ -1699,20 +1684,10 @@ static int batch_pass(KvHandle* kv, int layer, int pos0, int K, float* xc, uint6
         i += n;
     }
     // 3-5. Attention of the K tokens (QK-norm, RoPE, exact appends, causal over the cache).
-    auto swap_workspaces = [&] {
-        if (!many) return;
-        std::swap(kv->prefill_ws, kv->many_ws);
-        std::swap(kv->prefill_ws_bytes, kv->many_ws_bytes);
-        std::swap(kv->prefill_part, kv->many_part);
-        std::swap(kv->prefill_part_bytes, kv->many_part_bytes);
-        kv->keep_outgrown = !kv->keep_outgrown;
-    };
-    swap_workspaces();
-    const int rc = enqueue_prefill(kv, layer, -1, pos0, K, true, reinterpret_cast<uint64_t>(qb),
-                                   reinterpret_cast<uint64_t>(kb), reinterpret_cast<uint64_t>(vb), 0,
-                                   reinterpret_cast<uint64_t>(attn), stream, false);
-    swap_workspaces();
-    if (rc) return rc;
+    if (int rc = enqueue_prefill(kv, layer, -1, pos0, K, true, reinterpret_cast<uint64_t>(qb),
+                                 reinterpret_cast<uint64_t>(kb), reinterpret_cast<uint64_t>(vb), 0,
+                                 reinterpret_cast<uint64_t>(attn), stream, false))
+        return rc;
     // 6. Output projection (+ bias), post-norm, residual scale and residual add.
     const float* post = vecp(LLMP_W_POST_ATTN_NORM);
     const DevWeight& wo = W[LLMP_W_O];
@@ -1974,26 +1949,20 @@ static int enqueue_prefill(KvHandle* kv, int layer, int src_layer, int pos0, int
         // captured call whose wide workspace would have to grow, or one that finds no memory for
         // it, takes the narrow path.
         const size_t wide_need = wide.ksplit > 0 ? std::max(wide.total(), narrow.total()) : 0;
-        const bool own = narrow.ws <= kv->prefill_ws_bytes && narrow.part <= kv->prefill_part_bytes;
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (wide_need > kv->wide_ws_bytes || !own) LLMP_HIP_CHECK(hipStreamIsCapturing(st, &cap), "hipStreamIsCapturing");
-        const bool eager = cap == hipStreamCaptureStatusNone;
-        if (wide_need > kv->wide_ws_bytes && eager &&
-            grow_workspace(kv, kv->wide_ws, kv->wide_ws_bytes, wide_need, true, st, "wide workspace") != LLMP_OK)
-            (void)hipGetLastError();
-        use_wide = wide.ksplit > 0 && wide.total() <= kv->wide_ws_bytes;
-        if (use_wide || (!own && !eager && narrow.total() <= kv->wide_ws_bytes)) {
-            ws = kv->wide_ws;
+        const bool own = narrow.ws <= kv->prefill_ws.bytes && narrow.part <= kv->prefill_part.bytes;
+        bool capturing;
+        if (int rc = stream_capturing(st, &capturing)) return rc;
+        if (!capturing) (void)try_grow_workspace(kv, kv->wide_ws, wide_need, st);
+        use_wide = wide.ksplit > 0 && wide.total() <= kv->wide_ws.bytes;
+        if (use_wide || (!own && capturing && narrow.total() <= kv->wide_ws.bytes)) {
+            kv->wide_ws.captured |= capturing;
+            ws = kv->wide_ws.mem;
             a.part_o = reinterpret_cast<float*>(static_cast<char*>(ws) + (use_wide ? wide.ws : narrow.ws));
         } else {
-            if (int rc = grow_workspace(kv, kv->prefill_ws, kv->prefill_ws_bytes, narrow.ws, kv->keep_outgrown, st,
-                                        "tile workspace"))
-                return rc;
-            if (int rc = grow_workspace(kv, kv->prefill_part, kv->prefill_part_bytes, narrow.part, kv->keep_outgrown,
-                                        st, "split workspace"))
-                return rc;
-            ws = kv->prefill_ws;
-            a.part_o = static_cast<float*>(kv->prefill_part);
+            if (int rc = grow_workspace(kv, kv->prefill_ws, narrow.ws, capturing, st, "tile workspace")) return rc;
+            if (int rc = grow_workspace(kv, kv->prefill_part, narrow.part, capturing, st, "split workspace")) return rc;
+            ws = kv->prefill_ws.mem;
+            a.part_o = static_cast<float*>(kv->prefill_part.mem);
         }
     }
     const PrefillNeed& plan = use_wide ? wide : narrow;

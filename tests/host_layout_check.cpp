@@ -1,5 +1,5 @@
-// CPU driver of the library's host-side layout code (llmplayer_amd/csrc/host_layout.h), built by
-// tests/test_host_sanitize.py with g++ under AddressSanitizer and UndefinedBehaviorSanitizer.
+// CPU driver of the library's host-side layout code (llmplayer_amd/csrc/host_layout.h, and the
+// workspaces of workspace.h), built by tests/test_host_sanitize.py with g++ under AddressSanitizer and UndefinedBehaviorSanitizer.
 // It reads one command per line on stdin and answers one line per command on stdout:
 //   repack TYPE ROWS COLS IN OUT      -> "planes off0 off1 off2 off3 pitch0 pitch1 pitch2 pitch3"
 //                                        (the packed bytes are written to OUT)
@@ -11,16 +11,22 @@
 //   range H N ROW K V QS              -> "ek0 .. ek(H-1) ev0 .. ev(H-1) eq0 .. eq(H-1)": range
 //                                        exponents of fp32 rows K, V ([N][H*ROW] floats) and of
 //                                        the Q8_0 rows QS (N*H*ROW int8 quants, then the scales)
+//   workspace BYTES OP...             -> per OP "result bytes outgrown frees", ';' between them: a
+//                                        workspace over BYTES bytes of memory; OP gN grows it to N,
+//                                        cN the same under capture, tN where it can do without
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <fstream>
 #include <iostream>
 #include <iterator>
+#include <map>
 #include <sstream>
 #include <string>
 #include <vector>
 
 #include "host_layout.h"
+#include "workspace.h"
 
 static std::vector<uint8_t> read_file(const std::string& path) {
     std::ifstream f(path, std::ios::binary);
@@ -31,6 +37,28 @@ static void write_file(const std::string& path, const void* p, size_t n) {
     std::ofstream f(path, std::ios::binary);
     f.write(static_cast<const char*>(p), (std::streamsize)n);
 }
+
+// Memory of a fixed size for Workspace::grow; real allocations, so that a use after free or a
+// double one is caught.
+struct CountedMemory {
+    size_t left;
+    int frees = 0;
+    std::map<void*, size_t> live;
+    llmp::Alloc alloc(size_t bytes, void** mem) {
+        if (bytes > left) return llmp::Alloc::no_memory;
+        *mem = std::malloc(bytes);
+        std::memset(*mem, 0x5A, bytes);
+        live[*mem] = bytes;
+        left -= bytes;
+        return llmp::Alloc::ok;
+    }
+    void release(void* mem) {
+        left += live.at(mem);
+        live.erase(mem);
+        std::free(mem);
+        ++frees;
+    }
+};
 
 int main() {
     std::string line;
@@ -61,6 +89,24 @@ int main() {
             write_file(heads, stage.data(), stage.size());
             write_file(back, again.data(), again.size());
             std::printf("ok\n");
+        } else if (cmd == "workspace") {
+            CountedMemory dev;
+            in >> dev.left;
+            llmp::Workspace w;
+            std::vector<void*> outgrown;
+            std::string op, sep;
+            while (in >> op) {
+                const size_t n = std::stoul(op.substr(1));
+                const int r = op[0] == 't' ? (w.try_grow(n, outgrown, dev) ? 0 : 1)
+                                           : (int)w.grow(n, op[0] == 'c', outgrown, dev);
+                for (void* p : outgrown) std::memset(p, 0xA5, dev.live.at(p));   // still allocated
+                if (w.mem) std::memset(w.mem, 0xA5, w.bytes);
+                std::printf("%s%d %zu %zu %d", sep.c_str(), r, w.bytes, outgrown.size(), dev.frees);
+                sep = ";";
+            }
+            std::printf("\n");
+            for (void* p : outgrown) dev.release(p);
+            if (w.mem) dev.release(w.mem);
         } else if (cmd == "plan") {
             int pos, window, splits;
             in >> pos >> window >> splits;

@@ -142,6 +142,56 @@ def test_graph_of_a_short_call_outlives_the_growth_of_the_scratch():
                 b.free()
 
 
+@pytest.mark.parametrize("n,block", [(17, True), (16, True), (33, True), (16, False)],
+                         ids=["17 tokens", "16 tokens", "33 tokens", "16 tokens, attention alone"])
+def test_graph_outlives_the_growth_of_the_split_workspace(n, block):
+    """A captured call after 200 rows (two or three key splits) replays what it computed after
+    16-token calls at later positions, whose many splits need larger partials, and after new
+    allocations of the partials' size."""
+    c, dim, pos0, last = _config(), 512, 200, 3900
+    rng = np.random.default_rng(31)
+    lw, _ = tbb._weights(c, dim, (gp.GGML_Q4_K,) * 4, rng)
+    x = rng.standard_normal((n, dim)).astype(np.float32)
+    proj = [rng.standard_normal(n * w).astype(np.float32) for w in (c.q_dim, c.kv_dim, c.kv_dim)]
+    with hfp.HipForwardPass(c, last + 16) as fp:
+        fp.setBlockConfig(dim)
+        fp.uploadLayerWeights(0, lw)
+        fp.kv.write(0, 0, *(rng.standard_normal((last, c.kv_dim)).astype(np.float32) for _ in range(2)))
+        qkv = [hfp.DeviceBuffer(a.nbytes) for a in proj]
+        buf = hfp.DeviceBuffer(n * max(dim, c.q_dim) * 4)
+        fill = []
+        try:
+            for b, a in zip(qkv, proj):
+                b.upload(a)
+
+            def put():
+                buf.upload(x if block else np.zeros((n, c.q_dim), np.float32))
+
+            def call(pos, k):
+                if block:
+                    _lib.call("llmp_attn_block_batch", fp.kv.handle, 0, pos, k, buf.ptr, 0)
+                else:
+                    _lib.call("llmp_attn_prefill_f32", fp.kv.handle, 0, pos, k, *(b.ptr for b in qkv), 0, buf.ptr, 0)
+            put()
+            call(pos0, n)
+            want = buf.download(np.float32)
+            g = C.c_uint64()
+            _lib.call("llmp_graph_begin", 0)
+            call(pos0, n)
+            _lib.call("llmp_graph_end", 0, C.byref(g))
+            for later in (900, 2000, last):
+                call(later, 16)
+                fill.append(hfp.DeviceBuffer(1 << 20))
+                fill[-1].upload(np.full(1 << 18, np.nan, np.float32))
+                put()
+                _lib.call("llmp_graph_launch", g.value, 0)
+                np.testing.assert_array_equal(buf.download(np.float32), want)
+            _lib.call("llmp_graph_destroy", g.value)
+        finally:
+            for b in qkv + [buf] + fill:
+                b.free()
+
+
 @pytest.mark.parametrize("first", [(0, 300), (900, 40)])
 def test_capture_beyond_the_prepared_workspaces_runs_in_groups(first):
     """A captured call of more tokens, or at a later position, than the eager calls before it had:

@@ -3,7 +3,7 @@ UndefinedBehaviorSanitizer:
 
 - llmplayer_amd/csrc/host_layout.h (GGUF weight repacking, the KV re-layout between the
   reference's [pos][n_kv_heads * row] arrays and the head-major device planes, the decode step
-  plan and the default split count), built with g++ into tests/host_layout_check.cpp and
+  plan and the default split count) and workspace.h (the growth of the workspaces), built with g++ into tests/host_layout_check.cpp and
   checked against the GGUF block layouts, numpy transposes and the step plan's invariants;
 - the oracle (oracle/attn_oracle.c, oracle/block_oracle.c) built with the same sanitizers
   (`make -C oracle asan`), under which tests/test_oracle.py and tests/test_block_oracle.py run
@@ -215,6 +215,25 @@ def test_kv_relayout_is_a_head_major_transpose(driver, H, n, row):
     np.testing.assert_array_equal(np.fromfile(heads, np.uint8).reshape(H, n, row),
                                   host.reshape(n, H, row).transpose(1, 0, 2))
     np.testing.assert_array_equal(np.fromfile(back, np.uint8).reshape(n, H * row), host)
+
+
+@pytest.mark.parametrize("memory,ops,want", [
+    # at least twofold; the smaller buffer is freed first (a third one would not fit beside them)
+    (300, "g100 g50 g120 g260", ["0 100 0 0", "0 100 0 0", "0 200 0 1", "0 260 0 2"]),
+    # kept where a captured call used it, whichever call grows it
+    (1000, "c100 g150 g150 g300", ["0 100 0 0", "0 200 1 0", "0 200 1 0", "0 400 1 1"]),
+    (1000, "g100 c40 c250", ["0 100 0 0", "0 100 0 0", "0 250 1 0"]),
+    # a later call of a captured buffer frees nothing either
+    (1000, "c100 g90 g101", ["0 100 0 0", "0 100 0 0", "0 200 1 0"]),
+    # short of twice: exactly what is needed; short of that: refused, nothing kept is lost
+    (250, "g100 g120 c130", ["0 100 0 0", "0 200 0 1", "0 200 0 1"]),
+    (250, "c100 g140 g160", ["0 100 0 0", "0 140 1 0", "1 0 1 1"]),
+    (250, "c100 c200 g140", ["0 100 0 0", "1 100 0 0", "0 140 1 0"]),
+    # what can be done without: refused once, then not asked for again; smaller sizes still grow
+    (250, "t100 t300 t300 t200 t300", ["0 100 0 0", "1 0 0 1", "1 0 0 1", "0 200 0 1", "1 200 0 1"]),
+])
+def test_workspace_growth(driver, memory, ops, want):
+    assert _run(driver[0], [f"workspace {memory} {ops}"]) == [";".join(want)]
 
 
 def test_step_plan_invariants(driver):
