@@ -7,6 +7,7 @@
 #include <cstdint>
 
 #include "host_layout.h"
+#include "prefill_plan.h"
 
 namespace llmp {
 
@@ -14,8 +15,6 @@ namespace llmp {
 constexpr int kMaxSplits = 1024;
 // Largest GQA group (query heads per KV head) any decode kernel ships.
 constexpr int kMaxGroup = 8;
-// Tokens per launch of the token-batched projections (the MFMA's N).
-constexpr int kTokBatch = 16;
 
 // Arguments of one split-K decode launch.  All pointers are device pointers.  The kernels
 // derive the step plan (window start, rows per split, effective splits, RoPE row) from the
@@ -98,24 +97,13 @@ hipError_t launch_prefill_tiles(const pk::PrefillArgs& a, int head_dim, void* ws
                                 int n_tiles, int row_end, hipStream_t stream);
 hipError_t launch_prefill_attn(const pk::PrefillArgs& a, int head_dim, int group, const void* ws,
                                int tile0, int n_tiles, int n_cu, int ksplit, hipStream_t stream);
-// Key splits of a prefill call (1 unless the query blocks alone leave CUs idle: short prompts
-// after a long cached prefix, speculative verification); ksplit > 1 writes partials to
-// a.part_o / a.part_ml ([ksplit][P][Hq][D] and [..][2] floats) and adds a combine launch.
-constexpr int kMaxPrefillSplits = 64;
-int prefill_key_splits(int P, int pos0, int window, int n_kv_heads, int group, int head_dim,
-                       int n_cu);
-// Keys per tile and bytes per tile image (per KV head) for head_dim; 0 if unsupported.
-int prefill_tile_keys(int head_dim);
-size_t prefill_tile_bytes(int head_dim);
+// (Key splits, tile keys and bytes: prefill_plan.h.  ksplit > 1 writes partials to a.part_o /
+// a.part_ml, [ksplit][P][Hq][D] and [..][2] floats, and adds a combine launch.)
 
 // The combine of ksplit > 1 partials (also made by launch_prefill_attn).
 hipError_t launch_prefill_combine(const pk::PrefillArgs& a, int head_dim, int ksplit, hipStream_t stream);
-// The wide path (prefill_wide_kernels.h): its key splits for a call, 0 where the call stays on
-// the kernels above; keys and bytes per tile image; and its launches (images into `ws`,
-// attention, and with ksplit > 1 the combine).
-int prefill_wide_splits(int P, int pos0, int window, int n_kv_heads, int group, int head_dim, int n_cu);
-int prefill_wide_tile_keys(int head_dim);
-size_t prefill_wide_tile_bytes(int head_dim);
+// The wide path's launches (prefill_wide_kernels.h): images into `ws`, attention, and with ksplit
+// > 1 the combine.
 hipError_t launch_prefill_wide(const pk::PrefillArgs& a, int head_dim, int group, void* ws, int tile0, int n_tiles,
                                int row_end, int n_cu, hipStream_t stream);
 

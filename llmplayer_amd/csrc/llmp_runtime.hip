@@ -1118,13 +1118,6 @@ int llmp_layer_norm_mode(uint64_t handle, int layer, int mode) {
 struct BatchLayout {
     size_t q, k, v, attn, o, sc, q8b, q8d, q8s, xs, total;
 };
-// Tokens from which the projections run as tiled products (proj_gemm_kernels.h): the whole call at
-// the 24/8/128 shape with Q4_K_M weights takes 130 us for 95 tokens in groups of 16 and about 1.15 us
-// more per token; tiled 178 us at 96 tokens and 180 at 200.
-constexpr int kGemmTokens = 136;
-// Tokens of one pass through the projections and the attention: bounds the scratch (about 120 MB
-// at the 24/8/128 shape) at no cost, since a pass this long fills the chip many times over.
-constexpr int kPassTokens = 2048;
 static BatchLayout batch_layout(const KvHandle* kv, int qd, int kvd, int tokens, bool post, bool q8) {
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const int dim = kv->blk_dim, wide = dim > qd ? dim : qd;
@@ -1419,28 +1412,8 @@ static int enqueue_prefill(KvHandle* kv, int layer, int src_layer, int pos0, int
 
 static int batch_pass(KvHandle* kv, int layer, int pos0, int K, float* xc, uint64_t stream);
 
-// What a multi-token attention call of n tokens needs on one of its two paths: its key tiles (from
-// the first query's window start, or 0, to the last new row), the key splits (0: the wide path does
-// not take the call), and the bytes of the tile images and of the split partials.
-struct PrefillNeed {
-    int TK, tile0, n_tiles, ksplit;
-    size_t ws, part;
-    size_t total() const { return ws + part; }
-};
-static PrefillNeed prefill_need(const KvHandle* kv, const LayerCfg& c, int pos0, int n, bool wide) {
-    const int D = kv->head_dim, Hkv = kv->n_kv_heads, window = layer_window(c);
-    PrefillNeed r{};
-    r.ksplit = wide ? prefill_wide_splits(n, pos0, window, Hkv * c.krep, c.kgroup, D, G().n_cu)
-                    : prefill_key_splits(n, pos0, window, Hkv * c.krep, c.kgroup, D, G().n_cu);
-    if (r.ksplit == 0) return r;
-    r.TK = wide ? prefill_wide_tile_keys(D) : prefill_tile_keys(D);
-    r.tile0 = (window > 0 ? std::max(0, pos0 - window + 1) : 0) / r.TK;
-    r.n_tiles = (pos0 + n - 1) / r.TK - r.tile0 + 1;
-    const size_t tiles = (size_t)Hkv * (size_t)r.n_tiles;
-    if (wide) r.ws = KvHandle::pad256(tiles * prefill_wide_tile_bytes(D));
-    else if (r.ksplit == 1) r.ws = tiles * prefill_tile_bytes(D);   // splits stage straight from the cache
-    if (r.ksplit > 1) r.part = (size_t)r.ksplit * (size_t)n * (size_t)c.n_heads * (size_t)(D + 2) * sizeof(float);
-    return r;
+static PrefillShape prefill_shape(const KvHandle* kv, const LayerCfg& c) {
+    return {kv->n_kv_heads, c.krep, c.kgroup, kv->head_dim, layer_window(c), G().n_cu};
 }
 
 // Whether work enqueued on the stream now is recorded into a graph.
@@ -1534,24 +1507,29 @@ int llmp_attn_block_batch(uint64_t handle, int layer, int pos0, int n_tokens, ui
     if (pass > kTokBatch) {
         bool capturing;
         if (int rc = stream_capturing(st, &capturing)) return rc;
-        const size_t need = batch_layout(kv, qd, kvd, pass, W[LLMP_W_POST_ATTN_NORM].mem != nullptr,
-                                         kv->blk_input == LLMP_INPUT_Q8_1).total;
+        const bool q8 = kv->blk_input == LLMP_INPUT_Q8_1;
+        const PrefillShape ps = prefill_shape(kv, c);
+        const size_t need = batch_layout(kv, qd, kvd, pass, W[LLMP_W_POST_ATTN_NORM].mem != nullptr, q8).total;
         if (capturing) {
-            bool fits = need <= kv->many_buf.bytes;
-            for (int t0 = 0; fits && t0 < n_tokens; t0 += pass) {
-                const int n = std::min(pass, n_tokens - t0);
-                const PrefillNeed w = prefill_need(kv, c, pos0 + t0, n, true), p = prefill_need(kv, c, pos0 + t0, n, false);
-                fits = (w.ksplit > 0 && w.total() <= kv->wide_ws.bytes) ||
-                       (p.ws <= kv->prefill_ws.bytes && p.part <= kv->prefill_part.bytes) || p.total() <= kv->wide_ws.bytes;
+            const PrefillHave have{kv->wide_ws.bytes, kv->prefill_ws.bytes, kv->prefill_part.bytes};
+            if (need <= kv->many_buf.bytes && batch_fits(ps, pos0, n_tokens, pass, q8, have))
+                kv->many_buf.captured = true;
+            else
+                pass = kTokBatch;
+            // Groups whose workspaces are missing fail here, before any part of them is enqueued.
+            for (int t0 = 0; pass == kTokBatch && t0 < n_tokens; t0 += pass) {
+                const int n = batch_together(std::min(pass, n_tokens - t0), q8);
+                if (n == 0 || prefill_fits(ps, pos0 + t0, n, have)) continue;
+                const PrefillNeed p = prefill_need(ps, pos0 + t0, n, false);
+                if (int rc = grow_workspace(kv, kv->prefill_ws, p.ws, true, st, "tile workspace")) return rc;
+                if (int rc = grow_workspace(kv, kv->prefill_part, p.part, true, st, "split workspace")) return rc;
             }
-            if (fits) kv->many_buf.captured = true;
-            else pass = kTokBatch;
         } else {
             // The attention workspaces of the same call in groups of 16, which a later captured
             // call may take (this one does without them).
             size_t ws = 0, part = 0;
             for (int t0 = 0; t0 < n_tokens; t0 += kTokBatch) {
-                const PrefillNeed p = prefill_need(kv, c, pos0 + t0, std::min(kTokBatch, n_tokens - t0), false);
+                const PrefillNeed p = prefill_need(ps, pos0 + t0, std::min(kTokBatch, n_tokens - t0), false);
                 ws = std::max(ws, p.ws);
                 part = std::max(part, p.part);
             }
@@ -1569,12 +1547,12 @@ int llmp_attn_block_batch(uint64_t handle, int layer, int pos0, int n_tokens, ui
 
 // One pass of llmp_attn_block_batch over K tokens (rows xc), within the handle's scratch.
 static int batch_pass(KvHandle* kv, int layer, int pos0, int K, float* xc, uint64_t stream) {
-    // A group of one token takes the single-token launches, which are faster for it (27 against 49
-    // us at C3), after the others: it attends to their rows.
+    // A group of one token takes the single-token launches, after the others: it attends to their
+    // rows.
     if (K == 1) return enqueue_block(kv, layer, pos0, 0, reinterpret_cast<uint64_t>(xc), 0, stream);
-    if (K % kTokBatch == 1 && (kv->blk_input == LLMP_INPUT_Q8_1 || K < kGemmTokens)) {
-        if (int rc = batch_pass(kv, layer, pos0, K - 1, xc, stream)) return rc;
-        return batch_pass(kv, layer, pos0 + K - 1, 1, xc + (size_t)(K - 1) * kv->blk_dim, stream);
+    if (const int n = batch_together(K, kv->blk_input == LLMP_INPUT_Q8_1); n < K) {
+        if (int rc = batch_pass(kv, layer, pos0, n, xc, stream)) return rc;
+        return batch_pass(kv, layer, pos0 + n, K - n, xc + (size_t)n * kv->blk_dim, stream);
     }
     const LayerCfg& c = kv->layers[(size_t)layer];
     const DevWeight* W = c.w;
@@ -1926,8 +1904,9 @@ static int enqueue_prefill(KvHandle* kv, int layer, int src_layer, int pos0, int
         a.qk_scale = scale * log2e;
     }
     hipStream_t st = pick_stream(stream);
-    const PrefillNeed narrow = prefill_need(kv, c, pos0, n_tokens, false);
-    const PrefillNeed wide = prefill_need(kv, c, pos0, n_tokens, true);
+    const PrefillShape ps = prefill_shape(kv, c);
+    const PrefillNeed narrow = prefill_need(ps, pos0, n_tokens, false);
+    const PrefillNeed wide = prefill_need(ps, pos0, n_tokens, true);
     bool use_wide = false;
     void* ws = nullptr;
     if (use_static) {

@@ -11,21 +11,6 @@ constexpr int kAppendThreads = 256;
 template <int D>
 constexpr int tile_threads() { return D == 96 ? 192 : 256; }
 
-// Launch shape of the attention kernel: one query head per wave (HPW 1, measured best at the
-// C5 shape: each wave's K/V fragments feed its MFMAs while occupancy stays at 4 waves/SIMD),
-// 16*NB query tokens per workgroup, at most 8 waves.  NB_BIG is used when the grid then still
-// holds two workgroups per CU, else NB_BIG/2 (short prompts).
-constexpr int nb_big(int G) { return G >= 8 ? 1 : (8 / G >= 4 ? 4 : 8 / G); }
-
-// Workgroups per key split: query blocks of 16*NB tokens times KV heads.
-inline int prefill_items(int P, int Hkv, int NB) { return ((P + 16 * NB - 1) / (16 * NB)) * Hkv; }
-
-// Query blocks per workgroup the launch uses for P tokens and group size G (see launch_attn_dg).
-inline int prefill_nb(int P, int Hkv, int G, int n_cu) {
-    const int nb = nb_big(G);
-    return (nb > 1 && prefill_items(P, Hkv, nb) < 2 * n_cu) ? nb / 2 : nb;
-}
-
 template <int D, int G, int NB>
 hipError_t launch_attn_dgn(const pk::PrefillArgs& a, const uint4* ws, int tile0, int n_tiles,
                            int ksplit, int n_cu, hipStream_t stream) {
@@ -138,25 +123,12 @@ hipError_t launch_prefill_append(const pk::PrefillArgs& a, int head_dim, hipStre
     }
 }
 
-int prefill_tile_keys(int head_dim) {
-    switch (head_dim) {
-    case 64: return pk::TileLds<64>::TK;
-    case 96: return pk::TileLds<96>::TK;
-    case 128: return pk::TileLds<128>::TK;
-    case 256: return pk::TileLds<256>::TK;
-    default: return 0;
-    }
+template <int D>
+constexpr bool tile_as_planned() {
+    return prefill_tile_keys(D) == pk::TileLds<D>::TK && prefill_tile_bytes(D) == sizeof(pk::TileLds<D>);
 }
-
-size_t prefill_tile_bytes(int head_dim) {
-    switch (head_dim) {
-    case 64: return sizeof(pk::TileLds<64>);
-    case 96: return sizeof(pk::TileLds<96>);
-    case 128: return sizeof(pk::TileLds<128>);
-    case 256: return sizeof(pk::TileLds<256>);
-    default: return 0;
-    }
-}
+static_assert(tile_as_planned<64>() && tile_as_planned<96>() && tile_as_planned<128>() && tile_as_planned<256>(),
+              "the plan's tiles are the kernels'");
 
 hipError_t launch_prefill_tiles(const pk::PrefillArgs& a, int head_dim, void* ws, int tile0,
                                 int n_tiles, int row_end, hipStream_t stream) {
@@ -168,21 +140,6 @@ hipError_t launch_prefill_tiles(const pk::PrefillArgs& a, int head_dim, void* ws
     case 256: return launch_tiles_d<256>(a, w, tile0, n_tiles, row_end, stream);
     default: return hipErrorInvalidValue;
     }
-}
-
-int prefill_key_splits(int P, int pos0, int window, int n_kv_heads, int group, int head_dim,
-                       int n_cu) {
-    const int TK = prefill_tile_keys(head_dim);
-    if (TK <= 0 || group <= 0) return 1;
-    const int items = prefill_items(P, n_kv_heads, prefill_nb(P, n_kv_heads, group, n_cu));
-    if (items >= n_cu) return 1;
-    // Key tiles of the last query (the heaviest workgroup's range, up to one block's spread).
-    const int last = pos0 + P - 1;
-    const int kbeg = window > 0 ? std::max(0, last - window + 1) : 0;
-    const int tiles = last / TK - kbeg / TK + 1;
-    int ks = (2 * n_cu + items - 1) / items;          // about two workgroups per CU
-    ks = std::min(ks, std::max(1, tiles / 2));        // at least two tiles per split
-    return std::max(1, std::min(ks, kMaxPrefillSplits));
 }
 
 hipError_t launch_prefill_attn(const pk::PrefillArgs& a, int head_dim, int group, const void* ws,

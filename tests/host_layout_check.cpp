@@ -1,5 +1,5 @@
-// CPU driver of the library's host-side layout code (llmplayer_amd/csrc/host_layout.h, and the
-// workspaces of workspace.h), built by tests/test_host_sanitize.py with g++ under AddressSanitizer and UndefinedBehaviorSanitizer.
+// CPU driver of the library's host-side code (the layouts of llmplayer_amd/csrc/host_layout.h, the
+// workspaces of workspace.h and the paths of prefill_plan.h), built by tests/test_host_sanitize.py with g++ under AddressSanitizer and UndefinedBehaviorSanitizer.
 // It reads one command per line on stdin and answers one line per command on stdout:
 //   repack TYPE ROWS COLS IN OUT      -> "planes off0 off1 off2 off3 pitch0 pitch1 pitch2 pitch3"
 //                                        (the packed bytes are written to OUT)
@@ -14,6 +14,11 @@
 //   workspace BYTES OP...             -> per OP "result bytes outgrown frees", ';' between them: a
 //                                        workspace over BYTES bytes of memory; OP gN grows it to N,
 //                                        cN the same under capture, tN where it can do without
+//   need HKV KREP GROUP D WINDOW POS N -> "ksplit images partials wide-ksplit wide-images wide-partials
+//                                        groups pairs blocks*heads" of a multi-token attention call
+//                                        on 256 CUs (the wide path's after the other's)
+//   fits HKV KREP GROUP D WINDOW POS N PASS Q8 WIDE IMAGES PARTIALS -> "0|1" (batch_fits)
+//   together K Q8                     -> "tokens" (batch_together)
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -26,6 +31,7 @@
 #include <vector>
 
 #include "host_layout.h"
+#include "prefill_plan.h"
 #include "workspace.h"
 
 static std::vector<uint8_t> read_file(const std::string& path) {
@@ -107,6 +113,27 @@ int main() {
             std::printf("\n");
             for (void* p : outgrown) dev.release(p);
             if (w.mem) dev.release(w.mem);
+        } else if (cmd == "need" || cmd == "fits") {
+            llmp::PrefillShape s{};
+            int pos, n;
+            in >> s.n_kv_heads >> s.krep >> s.group >> s.head_dim >> s.window >> pos >> n;
+            s.n_cu = 256;
+            if (cmd == "need") {
+                const llmp::PrefillNeed p = llmp::prefill_need(s, pos, n, false), w = llmp::prefill_need(s, pos, n, true);
+                const llmp::WidePlan l = llmp::wide_plan(n, pos, s.window, s.n_kv_heads * s.krep, s.group,
+                                                         s.head_dim == 256 ? 128 : s.head_dim, s.n_cu);
+                std::printf("%d %zu %zu %d %zu %zu %d %d %d\n", p.ksplit, p.ws, p.part, w.ksplit, w.ws, w.part,
+                            l.groups, l.pairs, l.items);
+            } else {
+                int pass, q8;
+                llmp::PrefillHave have{};
+                in >> pass >> q8 >> have.wide >> have.ws >> have.part;
+                std::printf("%d\n", llmp::batch_fits(s, pos, n, pass, q8 != 0, have) ? 1 : 0);
+            }
+        } else if (cmd == "together") {
+            int k, q8;
+            in >> k >> q8;
+            std::printf("%d\n", llmp::batch_together(k, q8 != 0));
         } else if (cmd == "plan") {
             int pos, window, splits;
             in >> pos >> window >> splits;

@@ -233,6 +233,46 @@ def test_capture_beyond_the_prepared_workspaces_runs_in_groups(first):
         assert np.abs(y - want).max() <= 1e-4
 
 
+@pytest.mark.parametrize("n", [17, 33])
+def test_captured_call_with_a_last_group_of_one_token(n):
+    """Captured after an eager call of 35 tokens at the same position, where n - 1 tokens take more
+    key splits than 35: replays equal to the eager call to rounding (in groups of 16 where the
+    larger partials are missing), and to each other."""
+    c = hfp.ModelConfig(24, 8, 128, 1, architecture=hfp.ARCH_LLAMA, rope_freq_base=500000.0)
+    dim, pos0 = 512, 8000
+    rng = np.random.default_rng(6)
+    lw, _ = tbb._weights(c, dim, (gp.GGML_Q4_K,) * 4, rng)
+    x = rng.standard_normal((35, dim)).astype(np.float32)
+    with hfp.HipForwardPass(c, pos0 + 35) as fp:
+        fp.setBlockConfig(dim)
+        fp.uploadLayerWeights(0, lw)
+        fp.kv.write(0, 0, *(rng.standard_normal((pos0, c.kv_dim)).astype(np.float32) for _ in range(2)))
+        buf = hfp.DeviceBuffer(x.nbytes)
+        try:
+            def call(k):
+                _lib.call("llmp_attn_block_batch", fp.kv.handle, 0, pos0, k, buf.ptr, 0)
+            buf.upload(x)
+            call(35)
+            g = C.c_uint64()
+            _lib.call("llmp_graph_begin", 0)
+            call(n)
+            _lib.call("llmp_graph_end", 0, C.byref(g))
+            buf.upload(x)
+            call(n)
+            want = buf.download(np.float32, n * dim)
+            got = []
+            for _ in range(3):
+                buf.upload(x)
+                _lib.call("llmp_graph_launch", g.value, 0)
+                got.append(buf.download(np.float32, n * dim))
+                call(35)
+            _lib.call("llmp_graph_destroy", g.value)
+        finally:
+            buf.free()
+    assert np.abs(got[0] - want).max() <= 1e-4   # the bar of the batched blocks
+    assert np.array_equal(got[1], got[0]) and np.array_equal(got[2], got[0])
+
+
 def test_a_layer_captured_before_it_ever_ran_takes_the_tiled_projections():
     """Two layers of the same weights: the captured call of the one that never ran replays, bit for
     bit, what the other's eager call computed."""

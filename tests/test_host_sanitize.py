@@ -3,7 +3,8 @@ UndefinedBehaviorSanitizer:
 
 - llmplayer_amd/csrc/host_layout.h (GGUF weight repacking, the KV re-layout between the
   reference's [pos][n_kv_heads * row] arrays and the head-major device planes, the decode step
-  plan and the default split count) and workspace.h (the growth of the workspaces), built with g++ into tests/host_layout_check.cpp and
+  plan and the default split count), workspace.h (the growth of the workspaces) and
+  prefill_plan.h (what a multi-token attention call needs of them), built with g++ into tests/host_layout_check.cpp and
   checked against the GGUF block layouts, numpy transposes and the step plan's invariants;
 - the oracle (oracle/attn_oracle.c, oracle/block_oracle.c) built with the same sanitizers
   (`make -C oracle asan`), under which tests/test_oracle.py and tests/test_block_oracle.py run
@@ -234,6 +235,61 @@ def test_kv_relayout_is_a_head_major_transpose(driver, H, n, row):
 ])
 def test_workspace_growth(driver, memory, ops, want):
     assert _run(driver[0], [f"workspace {memory} {ops}"]) == [";".join(want)]
+
+
+def _needs(exe, calls):
+    """(images, partials, wide total or 0) of each (hkv, krep, group, d, window, pos, n)."""
+    out = [list(map(int, l.split())) for l in _run(exe, ["need " + " ".join(map(str, c)) for c in calls])]
+    return [(f[1], f[2], f[4] + f[5] if f[3] else 0) for f in out]
+
+
+def test_a_captured_batch_is_sized_by_the_calls_it_makes(driver):
+    """33 tokens run as 32 and one, and 32 take more key splits than 33 would: after 8000 rows of
+    24/8/128 the partials of 33 tokens, or of 35, do not hold those of 32."""
+    exe, _ = driver
+    shape = (8, 1, 3, 128, 0)
+    need = {n: _needs(exe, [shape + (8000, n)])[0] for n in (16, 32, 33, 35)}
+    assert need[32][1] > need[35][1] > need[33][1] > 0
+    fits = lambda pos, n, have, q8=0: _run(exe, ["fits " + " ".join(map(str, shape + (pos, n, 2048, q8) + have))]) == ["1"]
+    assert not fits(8000, 33, (0, 0, need[35][1]))
+    assert not fits(8000, 33, (0, 0, need[32][1] - 1)) and fits(8000, 33, (0, 0, need[32][1]))
+    assert fits(8000, 35, (0, 0, need[35][1])) and fits(8000, 33, (need[32][1], 0, 0))
+    assert not fits(8000, 17, (0, 0, need[16][1] - 1)) and fits(8000, 17, (0, 0, need[16][1]))
+    assert fits(8000, 1, (0, 0, 0))       # a single-token call: no workspace of these
+    images, partials, _ = _needs(exe, [shape + (0, 160)])[0]   # the Q8_1 input's last token alone
+    assert fits(0, 161, (0, images, partials), 1)
+    assert _run(exe, ["together 33 0", "together 161 0", "together 161 1", "together 1 0", "together 32 1"]) == \
+        ["32", "161", "160", "0", "32"]
+
+
+def test_batch_fits_means_every_call_fits(driver):
+    """Over random shapes, positions and workspaces: batch_fits is what the single calls' needs say."""
+    exe, _ = driver
+    rng = np.random.default_rng(12)
+    cases = []
+    for _ in range(200):
+        hkv, krep, group, d = (int(rng.choice(a)) for a in ((1, 2, 8), (1, 1, 2), (1, 2, 3, 4, 8), (64, 96, 128, 256)))
+        shape = (hkv, krep, group, d, int(rng.choice([0, 0, 300])))
+        pos, n, q8 = int(rng.integers(0, 9000)), int(rng.integers(1, 400)), int(rng.integers(0, 2))
+        passes = int(rng.choice([16, 128, 2048]))
+        calls = []
+        for t in range(0, n, passes):
+            k = min(passes, n - t)
+            k = int(_run(exe, [f"together {k} {q8}"])[0]) if k % 16 == 1 else k
+            calls += [shape + (pos + t, k)] if k else []
+        cases.append((shape, pos, n, passes, q8, calls))
+    flat = _needs(exe, [c for case in cases for c in case[5]])
+    lines, want = [], []
+    for shape, pos, n, passes, q8, calls in cases:
+        need, flat = flat[:len(calls)], flat[len(calls):]
+        ws, part = (max([x[i] for x in need], default=0) for i in (0, 1))
+        wide = max([x[2] or x[0] + x[1] for x in need], default=0)
+        for have in ((wide, 0, 0), (0, ws, part), (0, ws, max(part - 1, 0)), (wide // 2, ws // 2, part // 2)):
+            lines.append("fits " + " ".join(map(str, shape + (pos, n, passes, q8) + have)))
+            want.append(all((x[2] and x[2] <= have[0]) or (x[0] <= have[1] and x[1] <= have[2])
+                            or x[0] + x[1] <= have[0] for x in need))
+    assert [l == "1" for l in _run(exe, lines)] == want
+    assert any(want) and not all(want)
 
 
 def test_step_plan_invariants(driver):
