@@ -304,8 +304,8 @@ int llmp_attn_prefill_shared(uint64_t handle, int layer, int src_layer, int pos0
  * inputs; attention runs on the same fp16 hi/lo MFMA path (K, Q, V and P each split into two
  * fp16 parts, ~2^-22 of each operand's magnitude).  Range: any finite input.  K and V rows are
  * scaled by their layer's range exponents (llmp_kv_create) and the queries of each 16-token block
- * by the exponent of their largest magnitude before the split, so values beyond fp16's 65504
- * keep that precision; scores of ~1e3 and more are then resolved to ~2^-21 of their magnitude
+ * of a head (in long chunks each query) by the exponent of their largest magnitude before the
+ * split, so values beyond fp16's 65504 keep that precision; scores of ~1e3 and more are then resolved to ~2^-21 of their magnitude
  * (fp32: 2^-24).  gate may be 0.  The bf16 entry points take the same path. */
 int llmp_attn_prefill_f32(uint64_t handle, int layer, int pos0, int n_tokens, uint64_t q,
                           uint64_t k, uint64_t v, uint64_t gate, uint64_t out, uint64_t stream);

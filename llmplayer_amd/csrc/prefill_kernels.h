@@ -460,14 +460,17 @@ __device__ __forceinline__ void load8_bf16(const unsigned short* p, float (&v)[8
 }
 
 // Query fragment of one lane for MFMA B operands of STEP rows (32: four lane groups of 16, 16:
-// two of 32): dims STEP*s + 8*grp + j of query token qi (clamped into range), head hq, as fp32 (or widened from bf16), QK-normed, rotated, scaled,
-// then split.  With every dim rotated a NEOX pair (d, d + D/2) sits in one lane (but for head_dim
-// 96 in steps of 32); otherwise each element reads its partner from the input and normalises it exactly as the partner's own
-// lane does.  (A branch and a load per element cost one round trip each: 700 tokens at the
-// 16/8/128 shape with QK-norm took 69.3 us per call, 37.8 without.)  The scaled queries of the wave are divided
-// by 2^eq before their split, eq the range exponent of the largest magnitude among them (0
-// below 2^15; wave-uniform, so the factor that restores the scores stays in scalar registers);
-// the scores are multiplied back.
+// two of 32): dims STEP*s + 8*grp + j of query token qi (clamped into range), head hq, as fp32 (or
+// widened from bf16), QK-normed, rotated, scaled, then split.  With every dim rotated a NEOX pair
+// (d, d + D/2) sits in one lane (but for head_dim 96 in steps of 32); otherwise each element reads
+// its partner from the input and normalises it exactly as the partner's own lane does.  (A branch
+// and a load per element cost one round trip each: 700 tokens at the 16/8/128 shape with QK-norm
+// took 69.3 us per call, 37.8 without.)  The scaled queries are divided by 2^eq before their split,
+// eq the range exponent of the largest magnitude (0 below 2^15), and the scores are multiplied back.
+// In steps of 32 the wave's queries, 16 tokens of one head, share eq, and the factor that restores
+// the scores stays in scalar registers; in steps of 16 each query has its own, since the columns of
+// a wave are of several heads: with one for all, queries of 1e9 in one head left the outputs of the
+// others off by 5e-4.
 template <int D, int STEP = 32>
 __device__ __forceinline__ void query_fragment(const PrefillArgs& a, int qi, int hq, int qpos,
                                                int grp, f16x8 (&qh)[D / STEP],
@@ -591,7 +594,12 @@ __device__ __forceinline__ void query_fragment(const PrefillArgs& a, int qi, int
             qf[s][j] = qf[s][j] * a.qk_scale;
             qmax = fmaxf(qmax, fabsf(qf[s][j]));
         }
-    eq = wave_max_int(dk::range_exp_of_bits(dk::abs_bits(qmax)));
+    if constexpr (STEP == 32) {
+        eq = wave_max_int(dk::range_exp_of_bits(dk::abs_bits(qmax)));
+    } else {   // the query's own: lanes l and l ^ 32 hold its two halves
+        qmax = dk::lane_step<32, true>(qmax);
+        eq = dk::range_exp_of_bits(dk::abs_bits(qmax));
+    }
     const float fq = pow2i(-eq);
 #pragma unroll
     for (int s = 0; s < KS; ++s) {

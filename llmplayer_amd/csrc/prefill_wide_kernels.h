@@ -343,7 +343,8 @@ void prefill_wide_kernel(PrefillArgs a, const uint4* __restrict__ ws, const unsi
         c = wide_cols(a, group, vkh, blk, wave, lane);
         int eq;
         query_fragment<D, 16>(a, c.tok, c.hq, c.qpos, lane >> 5, w.qh, w.ql, eq);
-        // fs = 2^(ek + eq): the factor that restores the scores' scale (prefill_attn2_kernel).
+        // fs = 2^(ek + eq): the factor that restores the scores' scale (prefill_attn2_kernel); eq is
+        // the column's own.
         fs = pow2i(min(ek + eq, 127));
 #pragma unroll
         for (int d = 0; d < T::DT; ++d) w.o[d] = floatx16{};

@@ -88,3 +88,25 @@ def test_wide_prefill_over_q8_rows_equals_dequantised_rows():
             dq.free()
             do.free()
     np.testing.assert_array_equal(got.reshape(-1), want)
+
+
+def test_wide_prefill_keeps_heads_and_tokens_apart_in_range():
+    """Queries of 1e9 in one head, and in some tokens of another, leave the rest of the outputs as
+    they are without them.  Bar: 2e-6, outputs of at most ~2 over sums of 2^-22 products; only the
+    shared running maxima of a wave may move."""
+    c = hfp.ModelConfig(24, 8, 128, 1, architecture=LLAMA, rope_freq_base=500000.0)
+    pos0, P, big = 2000, 300, np.float32(1e9)
+    rng = np.random.default_rng(1)
+    q, k, v = (rng.standard_normal((P, n), dtype=np.float32) for n in (c.q_dim, c.kv_dim, c.kv_dim))
+    rows = [rng.standard_normal((pos0, c.kv_dim), dtype=np.float32) for _ in range(2)]
+    scaled = np.zeros((P, 24), bool)
+    scaled[:, 3] = True
+    scaled[::7, 10] = True
+    q2 = (q.reshape(P, 24, 128) * np.where(scaled, big, np.float32(1))[..., None]).reshape(P, -1)
+    out = []
+    for x in (q, q2):
+        with hfp.HipForwardPass(c, pos0 + P) as fp:
+            fp.kv.write(0, 0, *rows)
+            out.append(fp.prefill(0, pos0, x, k, v).reshape(P, 24, 128))
+    assert np.isfinite(out[1]).all()
+    assert np.abs(out[0] - out[1])[~scaled].max() <= 2e-6
