@@ -12,6 +12,13 @@ hipError_t launch_ff(const tk::ProjGemmArgs& a, hipStream_t st) {
     return hipGetLastError();
 }
 
+// A format as the product takes it.
+template <class F> struct GemmFormat { using type = F; };
+template <> struct GemmFormat<tk::PQ4K> { using type = tk::GQ4K; };
+template <> struct GemmFormat<tk::PQ5K> { using type = tk::GQ5K; };
+template <> struct GemmFormat<tk::PQ5_1> { using type = tk::GQ5_1; };
+template <> struct GemmFormat<tk::PQ2_K> { using type = tk::GQ2_K; };
+
 template <class Fn>
 hipError_t with_format(int t, Fn fn) {
     switch (t) {
@@ -49,9 +56,16 @@ hipError_t launch_weight_range(const gk::WPlanes& w, int ggml_type, int rows, in
 
 int proj_gemm_steps(int cols) { return (cols + tk::kChunk - 1) / tk::kChunk * (tk::kChunk / 16); }
 
+namespace {
+int input_tiles(int n_tokens) { return (n_tokens + tk::kGemmToks - 1) / tk::kGemmToks * (tk::kGemmToks / 32); }
+// The input sums, behind the fragments.
+float* input_sums(const void* xs, int n_tokens, int steps) {
+    return reinterpret_cast<float*>(static_cast<uint4*>(const_cast<void*>(xs)) + (size_t)input_tiles(n_tokens) * steps * 128);
+}
+}  // namespace
+
 size_t proj_gemm_input_bytes(int n_tokens, int cols) {
-    const size_t tiles = ((size_t)n_tokens + tk::kGemmToks - 1) / tk::kGemmToks * (tk::kGemmToks / 32);
-    return tiles * (size_t)proj_gemm_steps(cols) * 128 * sizeof(uint4);
+    return (size_t)input_tiles(n_tokens) * (size_t)proj_gemm_steps(cols) * (128 * sizeof(uint4) + 32 * sizeof(float));
 }
 
 hipError_t launch_tok_split(const float* x, long long x_pitch, int cols, const float* norm_w, float eps, float* sc,
@@ -63,9 +77,9 @@ hipError_t launch_tok_split(const float* x, long long x_pitch, int cols, const f
     hipLaunchKernelGGL(tk::tok_scale_kernel<tk::kPrepThreads>, dim3(n_tokens), dim3(tk::kPrepThreads), 0, st, x,
                        x_pitch, cols, norm_w, eps, sc);
     const int steps = proj_gemm_steps(cols);
-    const int tiles = (n_tokens + tk::kGemmToks - 1) / tk::kGemmToks * (tk::kGemmToks / 32);
-    hipLaunchKernelGGL(tk::tok_split_kernel<256>, dim3(tiles, (steps + 15) / 16), dim3(256), 0, st, x, x_pitch, cols, norm_w,
-                       sc, n_tokens, steps, static_cast<uint4*>(xs));
+    hipLaunchKernelGGL(tk::tok_split_kernel<256>, dim3(input_tiles(n_tokens), (steps + 15) / 16), dim3(256), 0, st, x,
+                       x_pitch, cols, norm_w, sc, n_tokens, steps, static_cast<uint4*>(xs),
+                       input_sums(xs, n_tokens, steps));
     return hipGetLastError();
 }
 
@@ -80,13 +94,17 @@ hipError_t launch_proj_gemm(tk::ProjGemmArgs a, int first_type, int second_type,
     }
     a.tok_tiles = (a.K + tk::kGemmToks - 1) / tk::kGemmToks;
     a.steps = proj_gemm_steps(a.cols);
+    a.xsum = input_sums(a.xs, a.K, a.steps);
     if (second_type >= 0) {
         if (!proj_tok_pair_supported(first_type, second_type)) return hipErrorInvalidValue;
-        if (first_type == gk::kQ3_K) return launch_ff<tk::PQ3K, tk::PQ5K>(a, st);
-        if (first_type == gk::kQ5_K) return launch_ff<tk::PQ5K, tk::PQ6K>(a, st);
-        return launch_ff<tk::PQ4K, tk::PQ6K>(a, st);
+        if (first_type == gk::kQ3_K) return launch_ff<tk::PQ3K, tk::GQ5K>(a, st);
+        if (first_type == gk::kQ5_K) return launch_ff<tk::GQ5K, tk::PQ6K>(a, st);
+        return launch_ff<tk::GQ4K, tk::PQ6K>(a, st);
     }
-    return with_format(first_type, [&](auto f) { return launch_ff<decltype(f), decltype(f)>(a, st); });
+    return with_format(first_type, [&](auto f) {
+        using F = typename GemmFormat<decltype(f)>::type;
+        return launch_ff<F, F>(a, st);
+    });
 }
 
 }  // namespace llmp

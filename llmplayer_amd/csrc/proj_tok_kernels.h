@@ -108,6 +108,27 @@ __device__ __forceinline__ f16x8_t as_f8(const uint4& u) { return __builtin_bit_
 __device__ __forceinline__ uint4 f16x8_of(const float (&v)[8]) {
     return make_uint4(pk_f16(v[0], v[1]), pk_f16(v[2], v[3]), pk_f16(v[4], v[5]), pk_f16(v[6], v[7]));
 }
+// Eight values from the bytes of c0 (0-3) and c1 (4-7).
+__device__ __forceinline__ uint4 f16x8_of_bytes(unsigned c0, unsigned c1) {
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        v[e] = (float)((c0 >> (8 * e)) & 0xFFu);
+        v[4 + e] = (float)((c1 >> (8 * e)) & 0xFFu);
+    }
+    return f16x8_of(v);
+}
+// The same minus a zero point below 64 for bytes below 64, without a conversion: 512 + q is the fp16
+// number 0x6000 | 2 q, and zero_point_f16 the zero point's, twice.
+__device__ __forceinline__ unsigned zero_point_f16(float z) { return (0x6000u | 2u * (unsigned)z) * 0x10001u; }
+__device__ __forceinline__ uint4 f16x8_less(unsigned c0, unsigned c1, unsigned zero) {
+    c0 += c0;
+    c1 += c1;
+    const unsigned u[4] = {__builtin_amdgcn_perm(0x60606060u, c0, 0x04010400u), __builtin_amdgcn_perm(0x60606060u, c0, 0x04030402u),
+                           __builtin_amdgcn_perm(0x60606060u, c1, 0x04010400u), __builtin_amdgcn_perm(0x60606060u, c1, 0x04030402u)};
+    const f16x8_t v = as_f8(make_uint4(u[0], u[1], u[2], u[3])) - as_f8(make_uint4(zero, zero, zero, zero));
+    return __builtin_bit_cast(uint4, v);
+}
 // hi = fp16(v), lo = fp16(v - hi).  Each lo half comes from one mixed-precision FMA,
 // hi(f16) * -1 + v(f32), which forms the difference exactly and rounds it once to fp16 into
 // its half of the register (the bits of rounding the exact fp32 difference, 3 instructions per
@@ -172,33 +193,32 @@ struct PQ4K {
         r.q[1] = ldo<uint2>(qp, (unsigned)(sb * 128 + 64 * h + 32 + 8 * kq));
         r.h = ldo<u32x4>(rp(w, 1, row), (unsigned)sb * 16u);
     }
-    static __device__ __forceinline__ void table(const Raw& r, float* tab, int m, int kq, int ch) {
-        // sub-block s = 4h + kq of this row
-        const int s = 4 * (ch & 1) + kq;
+    // (scale, min) of block kq of the chunk
+    static __device__ __forceinline__ float2 entry(const Raw& r, int kq, int ch) {
+        // sub-block 4h + kq of this row: bytes kq of the head's three scale words, without a branch
+        // (one here cost the tiled product's loop its registers)
         const float d = h2f((unsigned short)(r.h[0] & 0xFFFF));
         const float dmin = h2f((unsigned short)(r.h[0] >> 16));
-        int sc, mn;
-        auto byte_of = [&](int i) { return (int)((r.h[i >> 2] >> (8 * (i & 3))) & 0xFF); };
-        if (s < 4) {
-            sc = byte_of(4 + s) & 63;
-            mn = byte_of(8 + s) & 63;
-        } else {
-            sc = (byte_of(8 + s) & 15) | ((byte_of(s) >> 6) << 4);
-            mn = (byte_of(8 + s) >> 4) | ((byte_of(4 + s) >> 6) << 4);
-        }
-        reinterpret_cast<float2*>(tab + m * TAB)[kq] = make_float2(d * (float)sc, dmin * (float)mn);
+        const unsigned x = (r.h[1] >> (8 * kq)) & 0xFFu, y = (r.h[2] >> (8 * kq)) & 0xFFu, z = (r.h[3] >> (8 * kq)) & 0xFFu;
+        const unsigned odd = 0u - (unsigned)(ch & 1);
+        const unsigned sc = (odd & ((z & 15u) | ((x >> 6) << 4))) | (~odd & (x & 63u));
+        const unsigned mn = (odd & ((z >> 4) | ((y >> 6) << 4))) | (~odd & (y & 63u));
+        return make_float2(d * (float)sc, dmin * (float)mn);
     }
-    static __device__ __forceinline__ void afrag(const Raw& r, int gi, uint4 (&a)[NA], int) {
+    static __device__ __forceinline__ void table(const Raw& r, float* tab, int m, int kq, int ch) {
+        reinterpret_cast<float2*>(tab + m * TAB)[kq] = entry(r, kq, ch);
+    }
+    // the eight quants, one to a byte
+    static __device__ __forceinline__ void codes(const Raw& r, int gi, int, unsigned& c0, unsigned& c1) {
         const uint2 q = r.q[gi >> 1];
         const int sh = 4 * (gi & 1);
-        const unsigned u0 = (q.x >> sh) & 0x0F0F0F0Fu, u1 = (q.y >> sh) & 0x0F0F0F0Fu;
-        float v[8];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            v[e] = (float)((u0 >> (8 * e)) & 0xFF);
-            v[4 + e] = (float)((u1 >> (8 * e)) & 0xFF);
-        }
-        a[0] = f16x8_of(v);
+        c0 = (q.x >> sh) & 0x0F0F0F0Fu;
+        c1 = (q.y >> sh) & 0x0F0F0F0Fu;
+    }
+    static __device__ __forceinline__ void afrag(const Raw& r, int gi, uint4 (&a)[NA], int kq) {
+        unsigned c0, c1;
+        codes(r, gi, kq, c0, c1);
+        a[0] = f16x8_of_bytes(c0, c1);
     }
 };
 
@@ -380,22 +400,20 @@ struct PQ5_1 {
         r.d = ldo<unsigned short>(rp(w, 2, row), bk);
         r.m = ldo<unsigned short>(rp(w, 3, row), bk);
     }
-    static __device__ __forceinline__ void table(const Raw& r, float* tab, int m, int kq, int) {
-        reinterpret_cast<float2*>(tab + m * TAB)[kq] = make_float2(h2f(r.d), -h2f(r.m));
+    static __device__ __forceinline__ float2 entry(const Raw& r, int, int) { return make_float2(h2f(r.d), -h2f(r.m)); }
+    static __device__ __forceinline__ void table(const Raw& r, float* tab, int m, int kq, int ch) {
+        reinterpret_cast<float2*>(tab + m * TAB)[kq] = entry(r, kq, ch);
     }
-    static __device__ __forceinline__ void afrag(const Raw& r, int gi, uint4 (&a)[NA], int kq) {
-        unsigned c0, c1;
+    static __device__ __forceinline__ void codes(const Raw& r, int gi, int kq, unsigned& c0, unsigned& c1) {
         split_codes(r.q[gi], kq, c0, c1);
         const unsigned h = r.qh[gi] >> (8 * kq);
         c0 |= gk::spread4(h & 15u) << 4;
         c1 |= gk::spread4((h >> 4) & 15u) << 4;
-        float v[8];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            v[e] = (float)((c0 >> (8 * e)) & 0xFFu);
-            v[4 + e] = (float)((c1 >> (8 * e)) & 0xFFu);
-        }
-        a[0] = f16x8_of(v);
+    }
+    static __device__ __forceinline__ void afrag(const Raw& r, int gi, uint4 (&a)[NA], int kq) {
+        unsigned c0, c1;
+        codes(r, gi, kq, c0, c1);
+        a[0] = f16x8_of_bytes(c0, c1);
     }
 };
 
@@ -486,21 +504,20 @@ struct PQ5K {
         r.qh = ldo<uint2>(rp(w, 2, row), (unsigned)((ch >> 1) * 32 + 8 * kq));
         r.h = ch & 1;
     }
+    static __device__ __forceinline__ float2 entry(const Raw& r, int kq, int ch) { return PQ4K::entry(r.q4, kq, ch); }
     static __device__ __forceinline__ void table(const Raw& r, float* tab, int m, int kq, int ch) {
         PQ4K::table(r.q4, tab, m, kq, ch);
     }
-    static __device__ __forceinline__ void afrag(const Raw& r, int gi, uint4 (&a)[NA], int) {
-        const uint2 q = r.q4.q[gi >> 1];
-        const int sh = 4 * (gi & 1), hb = 4 * r.h + gi;
-        const unsigned u0 = ((q.x >> sh) & 0x0F0F0F0Fu) | (((r.qh.x >> hb) & 0x01010101u) << 4);
-        const unsigned u1 = ((q.y >> sh) & 0x0F0F0F0Fu) | (((r.qh.y >> hb) & 0x01010101u) << 4);
-        float v[8];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            v[e] = (float)((u0 >> (8 * e)) & 0xFF);
-            v[4 + e] = (float)((u1 >> (8 * e)) & 0xFF);
-        }
-        a[0] = f16x8_of(v);
+    static __device__ __forceinline__ void codes(const Raw& r, int gi, int kq, unsigned& c0, unsigned& c1) {
+        PQ4K::codes(r.q4, gi, kq, c0, c1);
+        const int hb = 4 * r.h + gi;
+        c0 |= ((r.qh.x >> hb) & 0x01010101u) << 4;
+        c1 |= ((r.qh.y >> hb) & 0x01010101u) << 4;
+    }
+    static __device__ __forceinline__ void afrag(const Raw& r, int gi, uint4 (&a)[NA], int kq) {
+        unsigned c0, c1;
+        codes(r, gi, kq, c0, c1);
+        a[0] = f16x8_of_bytes(c0, c1);
     }
 };
 
@@ -576,12 +593,15 @@ struct PQ2_K {
         reinterpret_cast<float4*>(tab + m * TAB)[kq] =
             make_float4(d * (float)(b0 & 15u), dm * (float)(b0 >> 4), d * (float)(b1 & 15u), dm * (float)(b1 >> 4));
     }
+    static __device__ __forceinline__ void codes(const Raw& r, int gi, int, unsigned& c0, unsigned& c1) {
+        auto spread = [](unsigned b) { return (b | (b << 6) | (b << 12) | (b << 18)) & 0x03030303u; };   // 2 bits to a byte
+        c0 = spread(r.q[gi] & 0xFFu);
+        c1 = spread(r.q[gi] >> 8);
+    }
     static __device__ __forceinline__ void afrag(const Raw& r, int gi, uint4 (&a)[NA], int kq) {
-        const unsigned q = r.q[gi];
-        float v[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = (float)((q >> (8 * (e >> 2) + 2 * (e & 3))) & 3u);
-        const uint4 u = f16x8_of(v);
+        unsigned c0, c1;
+        codes(r, gi, kq, c0, c1);
+        const uint4 u = f16x8_of_bytes(c0, c1);
         const uint4 z = make_uint4(0u, 0u, 0u, 0u);
         a[0] = kq < 2 ? u : z;   // columns 0-15: sub-block 2gi
         a[1] = kq < 2 ? z : u;   // columns 16-31: sub-block 2gi + 1
