@@ -194,9 +194,10 @@ __global__ __launch_bounds__(NTHR) void tok_split_kernel(const float* x, long lo
                 wv[0] = w0.x; wv[1] = w0.y; wv[2] = w0.z; wv[3] = w0.w;
                 wv[4] = w1.x; wv[5] = w1.y; wv[6] = w1.z; wv[7] = w1.w;
             }
-            const float f = exp2_int((int)sc[2 * t + 1]);
+            // (x*w) * 2^e; a factor below 1 goes to x, whose product with w may exceed fp32's range.
+            const float f = exp2_int((int)sc[2 * t + 1]), fx = fminf(f, 1.0f), fv = fmaxf(f, 1.0f);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = (xv[e] * wv[e]) * f;
+            for (int e = 0; e < 8; ++e) v[e] = ((xv[e] * fx) * wv[e]) * fv;
         }
         uint4 h, l;
         split8(v, h, l);

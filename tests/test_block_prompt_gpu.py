@@ -79,6 +79,27 @@ def test_groups_of_16_in_one_launch_append_what_single_groups_append():
         np.testing.assert_array_equal(a, b)
 
 
+def test_prompt_inputs_near_the_largest_float():
+    """A token with a value whose product with the norm weight exceeds fp32's range, as its square
+    does: its RMSNorm factor is 0 and so are its V rows; those of the others stay bit for bit."""
+    c, dim, K = _config(), 512, 140
+    rng = np.random.default_rng(2)
+    lw, _ = tbb._weights(c, dim, (gp.GGML_Q4_K,) * 4, rng)
+    lw.attnNorm = np.full(dim, 1.5, np.float32)
+    x = rng.standard_normal((K, dim)).astype(np.float32)
+    rows = []
+    for big in (1.0, 3e38):
+        x[5, 7] = np.float32(big)
+        with hfp.HipForwardPass(c, K) as fp:
+            fp.setBlockConfig(dim)
+            fp.uploadLayerWeights(0, lw)
+            fp.uploadXBatch(x)
+            fp.forwardAttentionBlockBatch(0, 0, K)
+            rows.append(fp.kv.read(0, 0, K)[1])
+    assert (rows[1][5] == 0).all()
+    np.testing.assert_array_equal(np.delete(rows[0], 5, 0), np.delete(rows[1], 5, 0))
+
+
 @pytest.mark.parametrize("xs,ws", [(1e6, 1e-6), (1e-20, 1.0), (1.0, 3e4)])
 def test_prompt_far_from_fp16_range(xs, ws):
     """F32 projections: y = W x to 2^-18 of sum |W||x| per element, whatever their scales (fp32
