@@ -138,9 +138,13 @@ inline bool prefill_fits(const PrefillShape& s, int pos0, int n, const PrefillHa
 }
 
 // ---- passes of the attention half of many tokens (llmp_attn_block_batch) ---------------------------
-// Tokens from which the projections run as tiled products (proj_gemm_kernels.h): the whole call at
-// the 24/8/128 shape with Q4_K_M weights takes 130 us for 95 tokens in groups of 16 and about 1.15 us
-// more per token; tiled 178 us at 96 tokens and 180 at 200.
+// Tokens from which the projections run as tiled products (proj_gemm_kernels.h): about where the two
+// cross at the 24/8/128 shape.  Whole calls there, groups against tiled, us: Q4_K_M 144 tokens 174
+// against 184, 176 tokens 204 against 184; Q8_0 112 tokens 162 against 161; F32 80 tokens 162 against
+// 178.  In groups a token costs 45-90 us per G weights by format, tiled a call has 55 us and 18 us per
+// 1000 columns to spend first, so other widths cross elsewhere: 32/8/128 (dim 4096) at 50-90 tokens,
+// 32/8/64 (dim 2048) at 110-170, but 16/8/128 (dim 1024) at 190-280 (144 tokens in Q4_K_M 86 against
+// 122) and 4/1/256 (dim 1152) at 340-420 (144 tokens in Q8_0 61 against 97).
 constexpr int kGemmTokens = 136;
 // Tokens of one pass through the projections and the attention: bounds the scratch (about 120 MB
 // at the 24/8/128 shape) at no cost, since a pass this long fills the chip many times over.

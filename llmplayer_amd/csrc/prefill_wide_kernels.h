@@ -12,14 +12,14 @@
 // form, which had the LDS two thirds busy at the matrix peak.  Key tiles are written once per
 // call as images in operand order (each operand fragment one 1 KB run, lane l at 16 l): a tile
 // goes from L2 to LDS by global_load_lds, 16 bytes per lane, through no register, and every
-// operand read is a lane-linear ds_read_b128 (no bank conflicts).  32 KB per tile (64 keys at
-// head_dim 64, 32 keys at 96 and 128) in two buffers leave two workgroups per CU, so one
+// operand read is a lane-linear ds_read_b128 (no bank conflicts).  Tiles of 32 KB (64 keys at
+// head_dim 64, 32 keys at 128; 24 KB for 32 keys at 96) in two buffers leave two workgroups per CU, so one
 // workgroup's softmax runs under the other's products.
 //
 // Measured (MI355X, attention kernel by rocprof, 16x16 kernel before): 24/8/128, 8192 fp32 tokens
-// 1662 -> 1196 us (1.03 PFLOP/s of products issued; a library fp16 GEMM of 8192^3 reaches 1.20 on
+// 1662 -> 1172 us (1.05 PFLOP/s of products issued; a library fp16 GEMM of 8192^3 reaches 1.20 on
 // the same card, where the clock falls to about 1.6 GHz under either); 32/8/64, 2048 bf16 tokens
-// 66.6 -> 59.4 us; 16/8/128, 777 tokens after 1501 rows 118 -> 63.5 us.  Steering the schedule
+// 66.6 -> 59.1 us; 16/8/128, 777 tokens after 1501 rows 118 -> 63.7 us.  Steering the schedule
 // (operand reads three products ahead, independent accumulators in turn, wave priorities)
 // measured no faster at any of the three.
 //
