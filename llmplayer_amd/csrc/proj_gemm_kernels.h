@@ -11,7 +11,7 @@
 // Bound: neither memory nor the matrix units (a fifth busy) nor the vector units (a third), but the
 // chain of a stage (operand reads, products beside the next group's decoding and the scaling, fragment
 // writes, barrier) and the workgroup count: 640 for Q/K/V and 384 for Wo on 512 slots at 1000 tokens
-// of that shape, where they take 158 and 108 us (64 and 39 GFLOP of products), against 1370 and 750 us
+// of that shape, where they take 160 and 108 us (64 and 39 GFLOP of products), against 1370 and 750 us
 // in groups.  A 128 x 128 tile of 8 waves took 196 and 109 us where this one took 170 and 113 (with
 // weights in two parts, then), and 226 against 178 us for the whole call at 96 tokens.
 //
@@ -536,7 +536,9 @@ __device__ __forceinline__ void gemm_rows(const ProjGemmArgs& a, const GemmSeg& 
 #pragma unroll
                 for (int i = 0; i < 4 * kGemmStage; ++i) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // a product
-                    __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);   // decoding, scaling
+                    // decoding, scaling (with a min 4: 200 tokens in Q4_K 178.8 us, 182.4 with 8; without, 165
+                    // against 166.9 in Q8_0)
+                    __builtin_amdgcn_sched_group_barrier(0x002, F::MIN ? 4 : 8, 0);
                 }
             } else {
                 __builtin_amdgcn_sched_barrier(0);
